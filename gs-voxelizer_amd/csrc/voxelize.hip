@@ -180,6 +180,24 @@ __device__ __forceinline__ bool may_touch(float mx, float my, float mz, float a,
     return !(sm * (sm - K) > r * 1.001f + 0.01f);  // NaN anywhere -> comparisons false -> keep
 }
 
+// The exp2 of three values, issued back to back at a raised wave priority.  A
+// SIMD pairs two waves' wave64 VALU instructions (~2.2 cycles each instead of
+// 4 to 6), and a v_exp_f32 (8 cycles) among them breaks the pairing for many of
+// the instructions that follow.  A timing probe of the backward's plane of rows
+// (473 VALU, 24 v_exp_f32, 16 LDS reads; SIMD-cycles at 4 waves per SIMD): 1,606
+// as compiled, 1,495 with an s_nop every 16 instructions, 1,338 with each row's
+// three v_exp_f32 together between priority changes, 1,189 with the v_exp_f32
+// replaced by moves.  k_vox_bwd: 336 -> 324 us at 256^3 / 200k, 133 -> 121 us at
+// 100 x 150 x 80 / 100k, 2.63 -> 2.54 ms at 512^3 / 1M.  The asm statements tie
+// the order to the values.
+__device__ __forceinline__ void exp2_together(float &x, float &y, float &z) {
+    asm volatile("s_setprio 3" : "+v"(x), "+v"(y), "+v"(z));
+    x = __builtin_amdgcn_exp2f(x);
+    y = __builtin_amdgcn_exp2f(y);
+    z = __builtin_amdgcn_exp2f(z);
+    asm volatile("s_setprio 0" : "+v"(x), "+v"(y), "+v"(z));
+}
+
 // x + y, never contracted with a product that feeds it: the operand is a
 // separately rounded (and, below 2^-126, flushed) binary32 product.
 __device__ __forceinline__ float add_nc(float x, float y) {
@@ -839,9 +857,10 @@ __device__ __forceinline__ void pair_moments(const float4 *s_rows, float mxl, fl
             if (kChain) {
                 // E_u = q + 2 u_r x_u (2 x_u and 2 al are exact doublings)
                 const float q = fmaf(-ur, ur, cr);
-                const float step = __builtin_amdgcn_exp2f(ur * (2.0f * f.al));      // 2^(2 al u_r)
-                float e1 = __builtin_amdgcn_exp2f(fmaf(ur, 2.0f * xu[0], q));  // u = 0
-                float e2 = __builtin_amdgcn_exp2f(fmaf(ur, 2.0f * xu[4], q));  // u = 4
+                float step = ur * (2.0f * f.al);       // 2^(2 al u_r)
+                float e1 = fmaf(ur, 2.0f * xu[0], q);  // u = 0
+                float e2 = fmaf(ur, 2.0f * xu[4], q);  // u = 4
+                exp2_together(step, e1, e2);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     sv[k] = e1 * G[k];
