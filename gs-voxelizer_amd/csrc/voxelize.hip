@@ -269,21 +269,41 @@ __device__ __forceinline__ int8_t l1_sign(float v, float t) {
 template <int C>
 constexpr int kRecF4 = (13 + C + 3) / 4;
 
+// Orders one wave's LDS writes before its own later reads (a wave's LDS accesses
+// execute in order): the batch loop's barrier where waves of a workgroup walk
+// lists of different lengths.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // Six waves per SIMD at C = 1 (78 VGPRs, no spills; 3 us faster at cfg3 than
 // five); more channels would spill at six.
-template <int C>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, 8))) void k_vox_fwd(
+//
+// S waves per tile (fwd_split chooses S), each walking an equal share of the
+// tile's list, at least kMinShare pairs; wave 0 adds their sums in order and
+// writes the tile.
+constexpr int kMinShare = 16;  // 12 to 32 measured alike
+
+template <int C, int S>
+__global__ __launch_bounds__(kWave *S)
+__attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, 8))) void k_vox_fwd(
     int D, int H, int W, int Tx, int Ty, int64_t T, int n, int n_isect,
     const int *__restrict__ ids, const int2 *__restrict__ bins, const float4 *__restrict__ pos_radii,
     const float2 *__restrict__ conics, const float *__restrict__ intens, float *__restrict__ vol,
     const float *__restrict__ target, float *__restrict__ tile_loss, int8_t *__restrict__ sgn,
     uint8_t *__restrict__ pair_live, uint64_t *__restrict__ wave_rec, int wave_cap) {
-    __shared__ float4 s_rec[kWave][kRecF4<C>];
+    // a wave's records, and (S > 1) its sums: 2C float4 a lane
+    constexpr int kLaneF4 = S > 1 && 2 * C > kRecF4<C> ? 2 * C : kRecF4<C>;
+    __shared__ float4 s_all[S][kWave * kLaneF4];
     const int64_t tile = xcd_runs(blockIdx.x);
     if (tile >= T) return;
-    const int lane = threadIdx.x;
+    const int lane = S == 1 ? threadIdx.x : threadIdx.x & (kWave - 1);
+    const int wave = S == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    float4(*const s_rec)[kRecF4<C>] = reinterpret_cast<float4(*)[kRecF4<C>]>(s_all[wave]);
     const bool timeline = wave_rec != nullptr && (int64_t)blockIdx.x < wave_cap;
-    if (timeline && lane == 0) {
+    if (timeline && threadIdx.x == 0) {
         wave_rec[3 * (int64_t)blockIdx.x] = wall_clock64();
         wave_rec[3 * (int64_t)blockIdx.x + 2] = (uint64_t)tile;
     }
@@ -293,6 +313,14 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(C == 1 ? 
     int2 range = bins[tile];
     range.x = max(range.x, 0);
     range.y = min(range.y, n_isect);  // never index past the id array
+    int sharing = 1;  // waves with pairs of this tile
+    if (S > 1) {      // (a range may be empty or reversed)
+        const int len = max(range.y - range.x, 0), end = range.y;
+        const int64_t share = max((len + S - 1) / S, kMinShare);
+        sharing = (int)((len + share - 1) / share);
+        range.y = (int)min<int64_t>(end, range.x + (wave + 1) * share);
+        range.x = (int)min<int64_t>(end, range.x + wave * share);
+    }
 
     float acc[GSV_TILE][C];
 #pragma unroll
@@ -421,7 +449,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(C == 1 ? 
         uint64_t cmask = chain_mask & ~omask;
         uint64_t fmask = fast_mask & ~chain_mask;
         uint64_t smask = live_mask & ~fast_mask;
-        __syncthreads();
+        if (S == 1) __syncthreads(); else wave_sync();
         // One-way and centre-out chained Gaussians, then the other gate-free
         // ones, then the exact-gate ones of the batch: single-path loops keep the
         // accumulators in place (no copies per trip).
@@ -536,7 +564,29 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(C == 1 ? 
                 for (int c = 0; c < C; ++c) acc[u][c] = fmaf(a, iw[c], acc[u][c]);
             }
         }
+        if (S == 1) __syncthreads(); else wave_sync();
+    }
+    if (S > 1) {
+        constexpr int kN = 2 * C;  // float4 of a lane's sums
+        if (wave > 0 && wave < sharing) {
+#pragma unroll
+            for (int q = 0; q < kN; ++q) {
+                float v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = acc[(4 * q + k) / C][(4 * q + k) % C];
+                s_all[wave][q * kWave + lane] = make_float4(v[0], v[1], v[2], v[3]);
+            }
+        }
         __syncthreads();
+        if (wave > 0) return;
+        for (int w = 1; w < sharing; ++w)
+#pragma unroll
+            for (int q = 0; q < kN; ++q) {
+                const float4 t = s_all[w][q * kWave + lane];
+                const float v[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) acc[(4 * q + k) / C][(4 * q + k) % C] += v[k];
+            }
     }
     if (C == 1) {
 #pragma unroll
@@ -1988,6 +2038,27 @@ bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) %
 namespace gsv {
 namespace {
 
+// Waves per tile of the forward: with one, a volume of few tiles leaves most of
+// the chip's ~6,000 wave slots empty and its time is one tile's list, walked by
+// one wave.  The largest power of two that keeps the launch within about two
+// rounds of the slots and no more waves than Gaussians: an average Gaussian
+// reaches ~8 tiles and more, so their shares then average 8 pairs and more.  The
+// rule takes nothing that differs between a count read on the host and one left
+// on the device, so the sums (their order depends on S and on the list alone)
+// are the same bits in both modes.  us at S = 1, 2, 4, 8 without the Gaussian
+// rule: 150 tiles of 103 pairs (2k Gaussians) 26.8, 18.5, 12.5, 10.6; 2,470 of
+// 495 (100k) 117, 94, 82, 84; 4,096 of 81 (50k) 35.5, 30.1, 31.9, 39.9; 2,470 of
+// 20 (5k) 14.0, 14.0, 16.5, 22.1; 11,960 of 143 (C = 3, 120k) 133, 132, 137, 189;
+// 32,768 of 108 (200k) 178, 178, 194, 275.
+constexpr int64_t kSplitWaves = 12288;
+constexpr int kMaxSplit = 16;
+
+int fwd_split(int64_t T, int64_t n) {
+    int split = 1;
+    while (split < kMaxSplit && 2 * split * T <= kSplitWaves && 2 * split * T <= n) split *= 2;
+    return split;
+}
+
 // Forward; with `target`, also the L1 loss mean|volume - target| into *loss
 // (tile_loss: T floats of scratch) and sgn(volume - target) into sgn.
 int voxelize_fwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t n,
@@ -2008,13 +2079,19 @@ int voxelize_fwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t
     if (!empty && (!aligned(pos3d_radii, 16) || !aligned(conics, 8))) return GSV_ERR_INVALID_ARGUMENT;
     // an empty list still runs the kernel for the loss: every tile range is empty
     const int ni = empty ? 0 : (int)num_intersects;
-    const dim3 grid((unsigned)xcd_runs_grid(T)), block(kWave);
+    const dim3 grid((unsigned)xcd_runs_grid(T));
+    const int split = fwd_split(T, n);
     int wave_cap = 0;
     uint64_t *wave_rec = wave_timeline_buffer(&wave_cap);
     {
         KernelTimer timer(kTimedVoxFwd, s);
 #define GSV_VF(CH)                                                                                 \
-    hipLaunchKernelGGL(k_vox_fwd<CH>, grid, block, 0, s, D, H, W, Tx, Ty, T, n, ni, ids,           \
+    hipLaunchKernelGGL((split == 16  ? k_vox_fwd<CH, 16>                                           \
+                        : split == 8 ? k_vox_fwd<CH, 8>                                            \
+                        : split == 4 ? k_vox_fwd<CH, 4>                                            \
+                        : split == 2 ? k_vox_fwd<CH, 2>                                            \
+                                     : k_vox_fwd<CH, 1>),                                          \
+                       grid, dim3((unsigned)(kWave * split)), 0, s, D, H, W, Tx, Ty, T, n, ni, ids, \
                        reinterpret_cast<const int2 *>(tile_bins),                                  \
                        reinterpret_cast<const float4 *>(pos3d_radii),                              \
                        reinterpret_cast<const float2 *>(conics), intensities, volume, target,      \

@@ -338,3 +338,28 @@ def test_backward_gaussians_without_pairs_get_zero_gradients(device, mode):
         assert (a[outside.numpy()] == 0).all(), nm
         if mode == "pairs":  # float atomics leave the last bits to the schedule
             np.testing.assert_array_equal(a[rest], b[rest], err_msg=nm)
+
+
+@pytest.mark.parametrize("channels", [1, 2, 3, 4])
+@pytest.mark.parametrize("vol,n", [((8, 8, 8), 1), ((8, 8, 8), 15), ((8, 8, 8), 17),
+                                   ((8, 8, 8), 257), ((9, 17, 23), 24), ((9, 17, 23), 700),
+                                   ((24, 24, 24), 54), ((33, 31, 30), 2100)])
+def test_forward_waves_sharing_a_tile(device, vol, n, channels):
+    """Few tiles, so several waves share one tile's list (2 to 16 by the tile and
+    Gaussian counts; at least 16 pairs each): lists shorter than one share, of one
+    pair more than a share or a batch of 64, and ragged edge tiles.  Sums of up to
+    700 binary32 terms in another order differ by at most 700 * 2^-24 = 4e-5 of
+    their size: inside the suite's rel 1e-4."""
+    import gs_voxelizer.cuda as _C
+    work = S.make_gaussians(small_config(1, n, vol=vol, channels=channels), seed=n + channels)
+    p = _prepare(work, device)
+    inten = work.intensities.numpy()
+    ref, amb = O.voxelize_fwd(vol, p["rids"], p["rbins"], p["rpr"], p["rcn"], inten, with_amb=True)
+    live = torch.empty(p["I"], device=device, dtype=torch.uint8)
+    out = _C.voxelize_forward(vol, p["ids"], p["bins"], p["pr"], p["cn"], p["w"].intensities,
+                              pair_live=live)
+    report_close("volume", np32(out), ref, RTOL, ATOL, amb)
+    # the lists in capacity-sized arrays give the same bits
+    pad = torch.cat([p["ids"], torch.zeros(3 * p["I"] + 64, device=device, dtype=torch.int32)])
+    again = _C.voxelize_forward(vol, pad, p["bins"], p["pr"], p["cn"], p["w"].intensities)
+    assert torch.equal(out, again)
