@@ -82,7 +82,9 @@ def parse():
 
 class KernelTimer:
     """Wraps native entry points of gs_voxelizer.cuda and records HIP events on
-    the current stream (the one the kernels are launched on) around each call."""
+    the current stream (the one the kernels are launched on) around each call.
+    While installed, steps take the Python autograd classes, which call those
+    entry points one at a time (the native nodes call the library directly)."""
 
     def __init__(self, module, names):
         import torch
@@ -94,6 +96,8 @@ class KernelTimer:
         self.active = False
 
     def install(self):
+        from gs_voxelizer import _native
+        self.plain, _native.plain = _native.plain, lambda *tensors: False
         for n in self.names:
             fn = self.orig[n]
 
@@ -110,6 +114,8 @@ class KernelTimer:
             setattr(self.module, n, wrapped)
 
     def uninstall(self):
+        from gs_voxelizer import _native
+        _native.plain = self.plain
         for n, fn in self.orig.items():
             setattr(self.module, n, fn)
 

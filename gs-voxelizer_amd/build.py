@@ -1,19 +1,23 @@
-"""Build libgsvox.so (gfx950) in-tree: ``python gs-voxelizer_amd/build.py``.
+"""Build libgsvox.so (gfx950) and the native autograd nodes in-tree:
+``python gs-voxelizer_amd/build.py``.
 
 hipcc compiles every ``csrc/*.hip`` for ``--offload-arch=gfx950`` and links one
 C-ABI shared library next to the Python package, where ``gs_voxelizer._lib``
 loads it.  No torch headers are involved, so the library is independent of the
-torch build's C++ ABI.
+torch build's C++ ABI.  csrc/autograd.cpp (host code, g++) is the part that does
+use them: a Python extension module, gs_voxelizer/_autograd.so.
 """
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "gs_voxelizer", "libgsvox.so")
+AUTOGRAD = os.path.join(HERE, "gs_voxelizer", "_autograd.so")
 SOURCES = ["scan.hip", "project.hip", "binning.hip", "voxelize.hip"]
 
 HIPCC_FLAGS = [
@@ -50,8 +54,25 @@ def _clean(text):
     return "\n".join(l for l in text.splitlines() if not any(k in l for k in noise))
 
 
+def autograd_command(out):
+    """The g++ command of the native autograd nodes against the installed torch."""
+    import torch
+    base = os.path.dirname(torch.__file__)
+    include = [os.path.join(base, "include"),
+               os.path.join(base, "include", "torch", "csrc", "api", "include"),
+               os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+               sysconfig.get_paths()["include"]]
+    return ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+             "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_autograd",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+            + ["-isystem" + d for d in include]
+            + [os.path.join(CSRC, "autograd.cpp"), "-o", out, "-L" + os.path.join(base, "lib"),
+               "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"])
+
+
 def build(verbose=False):
-    """Compile the library; returns its path. Always recompiles.
+    """Compile the library and the autograd module; returns the library's path.
+    Always recompiles.
 
     Each source is compiled to an object in its own hipcc process (they run
     concurrently; every translation unit is self-contained), then one link
@@ -59,7 +80,12 @@ def build(verbose=False):
     """
     flags = [f for f in HIPCC_FLAGS if f != "-shared"]
     with tempfile.TemporaryDirectory(dir=os.path.dirname(OUT)) as tmpdir:
-        procs = []
+        procs, tmp_autograd = [], os.path.join(tmpdir, "_autograd.so")
+        cmd = autograd_command(tmp_autograd)
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        procs.append(("autograd.cpp", None, subprocess.Popen(
+            cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
         for s in SOURCES:
             obj = os.path.join(tmpdir, os.path.splitext(s)[0] + ".o")
             cmd = [hipcc()] + flags + SOURCE_FLAGS.get(s, []) + ["-c", os.path.join(CSRC, s), "-o", obj]
@@ -75,9 +101,10 @@ def build(verbose=False):
                 failed.append(f"{s} ({pr.returncode}):\n{log}")
             elif verbose and log.strip():
                 print(log, flush=True)
-            objs.append(obj)
+            if obj:
+                objs.append(obj)
         if failed:
-            raise RuntimeError("hipcc failed: " + "\n".join(failed))
+            raise RuntimeError("build failed: " + "\n".join(failed))
         tmp = os.path.join(tmpdir, "libgsvox.so")
         cmd = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", tmp]
         if verbose:
@@ -86,6 +113,7 @@ def build(verbose=False):
         if res.returncode != 0:
             raise RuntimeError(f"hipcc link failed ({res.returncode}):\n{_clean(res.stdout + res.stderr)}")
         os.replace(tmp, OUT)
+        os.replace(tmp_autograd, AUTOGRAD)
     return OUT
 
 

@@ -1,0 +1,38 @@
+"""The native autograd nodes (csrc/autograd.cpp) and which calls may take them.
+
+Plain calls of ``optim_to_render`` and ``voxelize_gaussians`` (ordinary tensors,
+no transform or mode active) go to ``project`` and ``voxelize``, which return
+nothing for a call they do not take; the Python autograd classes then do it, and
+raise its errors.
+"""
+import ctypes
+
+import torch
+from torch.autograd import forward_ad
+
+from . import _autograd, _lib
+
+_ENTRIES = ("gsv_status_string", "gsv_last_hip_error", "gsv_project_fwd", "gsv_project_bwd",
+            "gsv_cumsum_bin_workspace_bytes", "gsv_cumsum_bin_and_sort_device_count",
+            "gsv_voxelize_fwd", "gsv_voxelize_fwd_l1_workspace_bytes", "gsv_voxelize_fwd_l1",
+            "gsv_voxelize_bwd_workspace_bytes", "gsv_voxelize_bwd", "gsv_voxelize_bwd_l1")
+_L = _lib.load()
+_autograd.bind({name: ctypes.cast(getattr(_L, name), ctypes.c_void_p).value for name in _ENTRIES})
+
+project = _autograd.project
+voxelize = _autograd.voxelize
+
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def plain(*tensors) -> bool:
+    """Whether every argument is an ordinary tensor and nothing watches or
+    transforms the call: no subclass, torch.func transform, forward-mode level,
+    trace, compilation, or dispatch or function mode.  (Saved-tensor hooks and
+    anomaly mode act on native nodes as on Python ones.)"""
+    for t in tensors:
+        if type(t) not in _PLAIN:
+            return False
+    return not (torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active()
+                or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+                or forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None)

@@ -10,6 +10,7 @@ from torch import Tensor
 from torch.autograd import Function
 
 import gs_voxelizer.cuda as _C
+from gs_voxelizer import _native
 
 
 def optim_to_render(
@@ -42,11 +43,20 @@ def optim_to_render(
         num_tiles_hit (N,): int32 number of tiles in the box.
     The int32 outputs carry no gradient; intensities get no gradient from here.
     """
+    pos3d, scale3d, quat = pos3d.contiguous(), scale3d.contiguous(), quat.contiguous()
+    intensities = intensities.contiguous()
+    if pos3d_radii_buffer is None and _native.plain(pos3d, scale3d, quat, intensities):
+        D, H, W = (int(v) for v in vol_size_voxel)
+        wz, wy, wx = (float(v) for v in vol_size_world)
+        cz, cy, cx = (float(v) for v in vol_center_pos)
+        out = _native.project(pos3d, scale3d, quat, intensities, D, H, W, wz, wy, wx, cz, cy, cx)
+        if out:
+            return tuple(out)
     return _OptimToRender.apply(
-        pos3d.contiguous(),
-        scale3d.contiguous(),
-        quat.contiguous(),
-        intensities.contiguous(),
+        pos3d,
+        scale3d,
+        quat,
+        intensities,
         vol_size_voxel,
         vol_size_world,
         vol_center_pos,

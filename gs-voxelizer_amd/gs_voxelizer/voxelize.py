@@ -22,6 +22,7 @@ from torch import Tensor
 from torch.autograd import Function
 
 import gs_voxelizer.cuda as _C
+from gs_voxelizer import _native
 
 _INT32_MAX = 2**31 - 1
 _capacity = {}  # device index -> intersection capacity of the speculative path
@@ -123,16 +124,46 @@ def voxelize_gaussians(
     Returns:
         (D, H, W, C) float32 volume.
     """
+    pos3d_radii, conics = pos3d_radii.contiguous(), conics.contiguous()
+    intensities = intensities.contiguous()
+    out = _native_voxelize(pos3d_radii, conics, intensities, vol_size_voxel, tile_min, tile_max,
+                           num_tiles_hit, None, use_per_gaussian_backward)
+    if out:
+        return out[0]
     return _VoxelizeGaussians.apply(
-        pos3d_radii.contiguous(),
-        conics.contiguous(),
-        intensities.contiguous(),
+        pos3d_radii,
+        conics,
+        intensities,
         vol_size_voxel,
         tile_min,
         tile_max,
         num_tiles_hit,
         use_per_gaussian_backward,
     )
+
+
+def _native_voxelize(pos3d_radii, conics, intensities, vol_size_voxel, tile_min, tile_max,
+                     num_tiles_hit, target, use_per_gaussian_backward):
+    """The plain steady-state call through the native nodes (the same launches at
+    the recorded capacity, the same count check): [volume], or [loss, volume]
+    with a target.  None where the Python class has to do it: the first call on
+    the device, GSV_SYNC_COUNT=1, graph capture, inputs that are not plain, no
+    pairs, or more than the capacity holds (which is raised here first)."""
+    tensors = (pos3d_radii, conics, intensities, tile_min, tile_max, num_tiles_hit)
+    if not _native.plain(*(tensors if target is None else tensors + (target,))):
+        return None
+    if not pos3d_radii.is_cuda or not _speculate():
+        return None
+    dev = pos3d_radii.device
+    cap = _capacity.get(dev.index)
+    if cap is None or torch.cuda.is_current_stream_capturing():
+        return None
+    D, H, W = (int(v) for v in vol_size_voxel)
+    count, out = _native.voxelize(*tensors, target, D, H, W, bool(use_per_gaussian_backward), cap,
+                                  _count_slot(dev))
+    if (count > cap and count <= _INT32_MAX) or (out and count < cap // 4):
+        _capacity[dev.index] = _grow(count)
+    return out
 
 
 def _bin_and_forward(num_gaussians, vol_size_voxel, tile_min, tile_max, num_tiles_hit, fwd):
@@ -287,15 +318,21 @@ def voxelize_gaussians_l1_loss(
     differentiable too; a gradient reaching it from other uses is added.
     The loss equals torch's up to float summation order.
     """
+    pos3d_radii, conics = pos3d_radii.contiguous(), conics.contiguous()
+    intensities, target = intensities.contiguous(), target.contiguous()
+    out = _native_voxelize(pos3d_radii, conics, intensities, vol_size_voxel, tile_min, tile_max,
+                           num_tiles_hit, target, use_per_gaussian_backward)
+    if out:
+        return tuple(out)
     return _VoxelizeL1.apply(
-        pos3d_radii.contiguous(),
-        conics.contiguous(),
-        intensities.contiguous(),
+        pos3d_radii,
+        conics,
+        intensities,
         vol_size_voxel,
         tile_min,
         tile_max,
         num_tiles_hit,
-        target.contiguous(),
+        target,
         use_per_gaussian_backward,
     )
 

@@ -34,7 +34,7 @@ setup(
     license="MIT",
     python_requires=">=3.9",
     packages=["gs_voxelizer"],
-    package_data={"gs_voxelizer": ["libgsvox.so"]},
+    package_data={"gs_voxelizer": ["libgsvox.so", "_autograd.so"]},
     install_requires=["torch", "numpy"],
     cmdclass={"build_py": BuildWithLibrary},
     distclass=BinaryDistribution,
