@@ -1006,6 +1006,14 @@ constexpr int kStageTilesVerySparse = C == 1 ? 8 : 6;  // < kVerySparsePairs
 constexpr int64_t kSparsePairs = 64;
 constexpr int64_t kVerySparsePairs = 24;
 
+// The most waves of pairs whose backward is one launch: the waves that are
+// resident at once at the up to 235 VGPRs of k_vox_bwd with kRows > 1.  us for the
+// pairs and the rest pass, as two launches and as one: 280 waves (40 x 48 x 36 /
+// 2k) 22.5, 20.0; 980 (100 x 150 x 80 / 5k) 40.1, 26.7; 760 (its C = 2 scene of
+// fixed scales) 48.0, 28.1.
+constexpr int64_t kSmallWaves = 2048;
+constexpr int kSmallRows = 2;
+
 // Whether the backward may take chained rows: on, unless GSV_BWD_CHAIN=0 is
 // set when the process first asks, or gsv_set_backward_chains(0) was called.
 // Read once per process, then kept here.
@@ -1841,16 +1849,23 @@ __device__ __forceinline__ void zero_partial(const BwdArgs &a, int64_t e) {
 // occupancy target is silenced.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wpass-failed"
-template <int C, int K>
+//
+// kRows > 1 (up to kSmallWaves waves): workgroup row r takes its wave's groups r,
+// r + kRows, ... of K tiles, and no rest launch follows.  So few waves leave the
+// chip part idle, and the groups past a wave's first then run beside it.  The
+// groups are the same ones, so the gradients are the same bits.
+template <int C, int K, int kRows>
 __global__ __launch_bounds__(kWave)
-__attribute__((amdgpu_waves_per_eu(C == 2 || C == 3 ? 2 : 1, 8))) void k_vox_bwd(BwdArgs a) {
+__attribute__((amdgpu_waves_per_eu((C == 2 || C == 3) && kRows == 1 ? 2 : 1, 8))) void k_vox_bwd(
+    BwdArgs a) {
     __shared__ float4 s_g[K * (kWave * 2 * C + 1)];
     bwd_counts(a);
     // XCD slabs sized by the live wave count (the grid may be sized for a
     // larger capacity), so every XCD gets an equal share; blocks past the
     // slabs would alias waves of other blocks and leave.  With a work list at
     // least one wave runs, for the culled pairs' zeros.
-    const bool zeros = a.order != nullptr && a.partial != nullptr;
+    const int row = kRows == 1 ? 0 : (int)blockIdx.y;
+    const bool zeros = a.order != nullptr && a.partial != nullptr && row == 0;
     const int64_t waves = ((int64_t)a.n_work + kWave - 1) / kWave;
     const int64_t W = zeros ? max<int64_t>(waves, 1) : waves;
     const int64_t per = xcd_per(W);
@@ -1870,14 +1885,19 @@ __attribute__((amdgpu_waves_per_eu(C == 2 || C == 3 ? 2 : 1, 8))) void k_vox_bwd
         uint64_t starts;
         int nslots;
         const bool slots = bwd_slots(a, p0, L, starts, nslots);
-        if (threadIdx.x == 0) a.rest_flag[wv] = slots && nslots > K;
-        if (slots) {
+        if (kRows == 1 && threadIdx.x == 0) a.rest_flag[wv] = slots && nslots > K;
+        if (slots && nslots > row * K) {
             bwd_gaussian(a, L);
             // one wave-uniform choice: gate-free unless a live lane needs the exact gate
             const bool wave_fast = __all(!L.live || L.fast);
             const bool any_live = __any(L.live);
-            if (any_live || a.partial != nullptr)
-                bwd_group<C, K>(a, L, starts, 0, wave_fast, any_live, s_g);
+            if (any_live || a.partial != nullptr) {
+                if (kRows == 1)
+                    bwd_group<C, K>(a, L, starts, 0, wave_fast, any_live, s_g);
+                else
+                    for (int g0 = row * K; g0 < nslots; g0 += kRows * K)
+                        bwd_group<C, K>(a, L, starts, g0, wave_fast, any_live, s_g);
+            }
         }
     }
     if (ze >= 0) zero_partial<C>(a, ze);
@@ -2172,6 +2192,8 @@ int voxelize_bwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t
     prep.tile_min = tile_min; prep.tile_max = tile_max; prep.cum = cum_tiles_hit;
     prep.rec = reinterpret_cast<float4 *>(ws + L.rec);
     const int nprep = (int)((n + kPrepThreads - 1) / kPrepThreads);
+    const int64_t waves = (num_intersects + kWave - 1) / kWave;
+    const bool small = waves <= kSmallWaves;
     if (!pair_live) {
         const dim3 pgrid((unsigned)nprep), pblock(kPrepThreads);
         switch (channels) {
@@ -2214,7 +2236,6 @@ int voxelize_bwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t
         order = ord;
         d_work = kept;
     }
-    const int64_t waves = (num_intersects + kWave - 1) / kWave;
     const int64_t per = xcd_per(waves);
     const dim3 grid((unsigned)(kXcds * per)), block(kWave);
     const float numel = (float)((int64_t)D * H * W * channels);
@@ -2241,19 +2262,25 @@ int voxelize_bwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t
 #define GSV_VB(CH)                                                                                  \
     {                                                                                               \
         KernelTimer timer(kTimedVoxBwd, s);                                                         \
-        if (very_sparse) {                                                                          \
-            hipLaunchKernelGGL((k_vox_bwd<CH, kStageTilesVerySparse<CH>>), grid, block, 0, s,       \
+        if (small) {                                                                                \
+            const dim3 rows(grid.x, kSmallRows);                                                    \
+            hipLaunchKernelGGL((very_sparse ? k_vox_bwd<CH, kStageTilesVerySparse<CH>, kSmallRows>  \
+                                : sparse    ? k_vox_bwd<CH, kStageTilesSparse<CH>, kSmallRows>      \
+                                            : k_vox_bwd<CH, kStageTiles<CH>, kSmallRows>),          \
+                               rows, block, 0, s, args);                                            \
+        } else if (very_sparse) {                                                                   \
+            hipLaunchKernelGGL((k_vox_bwd<CH, kStageTilesVerySparse<CH>, 1>), grid, block, 0, s,       \
                                args);                                                               \
             if (int st = check_launch()) return st;                                                 \
             hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTilesVerySparse<CH>>),                     \
                                dim3(kRestBlocks), block, 0, s, args);                               \
         } else if (sparse) {                                                                        \
-            hipLaunchKernelGGL((k_vox_bwd<CH, kStageTilesSparse<CH>>), grid, block, 0, s, args);   \
+            hipLaunchKernelGGL((k_vox_bwd<CH, kStageTilesSparse<CH>, 1>), grid, block, 0, s, args);   \
             if (int st = check_launch()) return st;                                                 \
             hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTilesSparse<CH>>), dim3(kRestBlocks),     \
                                block, 0, s, args);                                                  \
         } else {                                                                                    \
-            hipLaunchKernelGGL((k_vox_bwd<CH, kStageTiles<CH>>), grid, block, 0, s, args);         \
+            hipLaunchKernelGGL((k_vox_bwd<CH, kStageTiles<CH>, 1>), grid, block, 0, s, args);         \
             if (int st = check_launch()) return st;                                                 \
             hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTiles<CH>>), dim3(kRestBlocks), block, 0, \
                                s, args);                                                            \

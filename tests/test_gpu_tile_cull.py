@@ -268,3 +268,35 @@ def test_very_thin_gaussians_are_not_culled_from_tiles_they_reach(device):
     ref, amb = O.voxelize_fwd(vol, ids_np, np32(bins), pr, cn, inten, with_amb=True)
     report_close("very thin Gaussians: volume", np32(out), ref, 1e-4, 1e-6, bound=amb)
     assert ref[..., 0].max() > 0.3
+
+
+@pytest.mark.parametrize("channels,vol,n", [(1, (20, 30, 17), 1), (1, (20, 30, 17), 900),
+                                            (1, (100, 150, 80), 2500), (2, (64, 64, 64), 1500),
+                                            (3, (33, 31, 30), 800), (4, (64, 64, 64), 700)])
+def test_small_scene_backward_matches_the_rest_pass(device, set_chains, channels, vol, n):
+    """Scenes of few pairs take one launch for all groups of tiles; arrays sized for
+    more pairs take the rest pass.  Waves that span one tile to many (sparse
+    volumes).  Without chained rows a pair's partial does not depend on its group
+    (the capacity also sets the tiles staged at once): the same bits."""
+    import gs_voxelizer.cuda as _C
+    set_chains(False)
+    work = S.make_gaussians(small_config(1, n, vol=vol, channels=channels), seed=n).to(device)
+    cfg = work.cfg
+    pr, cn, tmin, tmax, nt = _C.optim_to_render_forward(n, work.pos3d, work.scale3d, work.quat,
+                                                        work.intensities, vol, cfg.world,
+                                                        cfg.center)
+    cum, total = _C.cumsum_tiles_hit(nt)
+    I = int(total.item())
+    assert 0 < I < 2048 * 64
+    g = torch.randn(vol + (channels,), device=device)
+    grads = []
+    for cap in (I, 2049 * 64):
+        ids, bins, tiles = _C.bin_and_sort_gaussians_device_count(n, cap, total, tmin, tmax, cum,
+                                                                  vol, return_tiles=True)
+        live = torch.empty(cap, device=device, dtype=torch.uint8)
+        _C.voxelize_forward(vol, ids, bins, pr, cn, work.intensities, pair_live=live)
+        grads.append(_C.voxelize_backward_per_gaussian(
+            vol, ids, bins, pr, cn, work.intensities, g, tmin, tmax, cum, tiles_sorted=tiles,
+            count_dev=total, pair_live=live))
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
