@@ -124,6 +124,13 @@ __device__ __forceinline__ Gate make_gate(float mean) {
     return g;
 }
 
+// Sylvester's criterion on the conic, in binary32.
+__device__ __forceinline__ bool positive_definite(float a, float b, float c, float d, float e,
+                                                  float f) {
+    const float det = a * (d * f - e * e) - b * (b * f - c * e) + c * (b * e - c * d);
+    return a > 0.f && a * d - b * b > 0.f && det > 0.f;
+}
+
 // Whether a live Gaussian may use the gate-free evaluation: bounded gate with
 // t2 >= -60, intensities whose weights I * 2^-off stay below 2^120, a finite
 // centre and a finite positive-definite conic (Sylvester's criterion), so that
@@ -135,8 +142,7 @@ __device__ __forceinline__ bool gate_free_ok(const Gate &g, float max_abs_i, flo
     if (!(max_abs_i * g.fscale <= 0x1p120f)) return false;
     if (!__builtin_isfinite(mx + my + mz) || !__builtin_isfinite(a + b + c + d + e + f))
         return false;
-    const float det = a * (d * f - e * e) - b * (b * f - c * e) + c * (b * e - c * d);
-    return a > 0.f && a * d - b * b > 0.f && det > 0.f;
+    return positive_definite(a, b, c, d, e, f);
 }
 
 // Conservative test: can the ellipsoid {d^T Q d <= K^2}, K^2 = 2 ln(mean*1e6),
@@ -196,6 +202,18 @@ __device__ __forceinline__ void exp2_together(float &x, float &y, float &z) {
     y = __builtin_amdgcn_exp2f(y);
     z = __builtin_amdgcn_exp2f(z);
     asm volatile("s_setprio 0" : "+v"(x), "+v"(y), "+v"(z));
+}
+
+// may_touch's second test for a whole tile about its centre, from m = c^T Q c and
+// the sum of |Q c|'s components (binary64, rounded): true when no voxel centre of
+// the tile can pass the gate.  At the volume's far faces the whole tile's box is
+// larger than its inside voxels' (more pairs are kept there).  The box test is
+// left out: it never fires on the projection's boxes, and a box it would reject
+// far from the ellipsoid this one rejects too.
+__device__ __forceinline__ bool misses_tile(float m, float n1, float t2) {
+    const float K = __builtin_amdgcn_sqrtf(-2.0f * kLn2 * t2) * 1.001f + 0.01f;
+    const float sm = __builtin_amdgcn_sqrtf(m);
+    return sm * (sm - K) > 3.5f * n1 * 1.001f + 0.01f;  // NaN anywhere -> false: keep
 }
 
 // x + y, never contracted with a product that feeds it: the operand is a
@@ -278,8 +296,8 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-// Six waves per SIMD at C = 1 (78 VGPRs, no spills; 3 us faster at cfg3 than
-// five); more channels would spill at six.
+// At least six waves per SIMD at C = 1 (66 VGPRs, no spills, so seven; five and
+// eight, at 64, measured within 1 % of it); more channels would spill at six.
 //
 // S waves per tile (fwd_split chooses S), each walking an equal share of the
 // tile's list, at least kMinShare pairs; wave 0 adds their sums in order and
@@ -346,9 +364,25 @@ __attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, 8))) void k_vox_fwd(
                 mean /= (float)C;
                 const Gate gt = make_gate(mean);
                 live = gt.live;
-                if (live && gt.bounded)
-                    live = may_touch(p.x, p.y, p.z, c01.x, c01.y, c23.x, c23.y, c45.x, c45.y, gt.t2,
-                                     tg.xlo, tg.xhi, tg.ylo, tg.yhi, tg.zlo, tg.zhi);
+                // centred offsets: delta = c - p', p' = local index - 3.5
+                const float cx = p.x - (float)tg.x0 - 4.0f;
+                const float cy = p.y - (float)tg.y0 - 4.0f, cz = p.z - (float)tg.z0 - 4.0f;
+                // Q c and c^T Q c in binary64: the culling test and the rows' terms
+                // about the tile centre are both formed from them (a batch's set-up
+                // is ~13 % of the kernel's VALU time, most of it binary64 at 4 cycles
+                // an instruction; formed apart, with the box test, k_vox_fwd took
+                // 173 us at 256^3 / 200k instead of 167, 1.35 ms at 512^3 / 1M
+                // instead of 1.29)
+                double nx = 0.0, ny = 0.0, nz = 0.0, m = 0.0;
+                if (live) {
+                    const double X = cx, Y = cy, Z = cz, b = c01.y, c = c23.x, e = c45.x;
+                    nx = fma((double)c01.x, X, fma(b, Y, c * Z));
+                    ny = fma(b, X, fma((double)c23.y, Y, e * Z));
+                    nz = fma(c, X, fma(e, Y, (double)c45.y * Z));
+                    m = fma(X, nx, fma(Y, ny, Z * nz));
+                    if (gt.bounded && positive_definite(c01.x, c01.y, c23.x, c23.y, c45.x, c45.y))
+                        live = !misses_tile((float)m, (float)(fabs(nx) + fabs(ny) + fabs(nz)), gt.t2);
+                }
                 if (live) {
                     // the gate-free rows expand the form about the tile centre, whose
                     // terms grow with the conic (~12 |q| at the tile's edge) and cancel
@@ -357,9 +391,6 @@ __attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, 8))) void k_vox_fwd(
                     fast = gate_free_ok(gt, max_abs, p.x, p.y, p.z, c01.x, c01.y, c23.x, c23.y,
                                         c45.x, c45.y) &&
                            fmaxf(c01.x, fmaxf(c23.y, c45.y)) <= kFwdFastConicMax;
-                    // centred offsets: delta = c - p', p' = local index - 3.5
-                    const float cx = p.x - (float)tg.x0 - 4.0f;
-                    const float cy = p.y - (float)tg.y0 - 4.0f, cz = p.z - (float)tg.z0 - 4.0f;
                     const float A2 = -0.5f * kLog2e * c01.x;
                     const float4 q1 = make_float4(-kLog2e * c01.y, -kLog2e * c23.x,
                                                   -0.5f * kLog2e * c23.y, -kLog2e * c45.x);
@@ -371,17 +402,14 @@ __attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, 8))) void k_vox_fwd(
                         //   T1 = t1 - B py - C pz,
                         //   T0 = t0 + ty py + tz pz + D py^2 + E py pz + F pz^2,
                         // t0 = the form at the tile centre, ty/tz its y/z slopes there.
-                        // Formed in binary64 and rounded once.
+                        // Formed in binary64 from the conic itself and rounded once.
                         // (t1, -B, -C, t0 | ty, tz, D, E | F, Q0, Q1, Q2 | Q3, I*2^-off ...),
                         // Q_k = A2 * uc_k^2 + off for the four |uc| = 0.5, 1.5, 2.5, 3.5
-                        const double X = cx, Y = cy, Z = cz;
-                        const double a2 = A2, bb = q1.x, cc = q1.y, dd = q1.z, ee = q1.w, ff = F;
-                        rec[0] = (float)(2.0 * a2 * X + bb * Y + cc * Z);
+                        constexpr double kL = 1.4426950408889634074;  // log2(e)
+                        const double t1 = -kL * nx, t0 = (-0.5 * kL) * m;
+                        rec[0] = (float)t1;
                         rec[1] = -q1.x; rec[2] = -q1.y;
-                        const double t0 = X * (a2 * X + bb * Y + cc * Z) + Y * (dd * Y + ee * Z) +
-                                          ff * Z * Z;
-                        const double ty = -(bb * X + 2.0 * dd * Y + ee * Z);
-                        const double tz = -(cc * X + ee * Y + 2.0 * ff * Z);
+                        const double ty = kL * ny, tz = kL * nz;
                         rec[6] = q1.z; rec[7] = q1.w;
                         rec[8] = F;
                         // Chained rows (the first two loops below) split s(u) into
@@ -409,7 +437,6 @@ __attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, 8))) void k_vox_fwd(
                         one_way = ceilf(7.0f * bound_t1) + 2.0f <= K;
                         chain = one_way || ceilf(4.0f * bound_t1) + 2.0f <= K;
                         const double at = one_way ? -3.5 : (chain ? 0.5 : 0.0);  // anchor uc
-                        const double t1 = 2.0 * a2 * X + bb * Y + cc * Z;
                         rec[3] = (float)(t0 - at * t1 + (chain ? (double)gt.off + (double)K : 0.0));
                         rec[4] = (float)(ty - at * (double)rec[1]);
                         rec[5] = (float)(tz - at * (double)rec[2]);
