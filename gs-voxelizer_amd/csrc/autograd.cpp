@@ -97,6 +97,21 @@ bool is_vector(const Tensor &t, at::ScalarType type, const at::Device &dev, int6
            t.device() == dev && t.dim() == 1 && t.size(0) == n && t.is_contiguous();
 }
 
+// A tensor that a backward reads, as it comes back from the saved-tensor hooks,
+// which may hand over any other one.
+Tensor unpacked(const Tensor &t, at::ScalarType type, const at::Device &dev, int64_t numel,
+                const char *what) {
+    TORCH_CHECK(t.defined() && t.layout() == at::kStrided && t.scalar_type() == type &&
+                    t.device() == dev && t.numel() == numel,
+                what, ": expected ", numel, " values of scalar type ", type, " on ", dev);
+    return t.contiguous();
+}
+
+// The device that a forward ran on, kept as its index.
+at::Device gpu(int64_t index) {
+    return at::Device(at::kCUDA, (at::DeviceIndex)index);
+}
+
 bool fits(int64_t D, int64_t H, int64_t W) {
     constexpr int64_t most = 1 << 20;
     return D > 0 && H > 0 && W > 0 && D <= most && H <= most && W <= most;
@@ -109,10 +124,12 @@ struct Projected {
 };
 
 struct Project : public torch::autograd::Function<Project> {
+    // The intensities get no gradient from here, but make the outputs require one.
     static variable_list forward(AutogradContext *ctx, const Tensor &pos, const Tensor &scale,
-                                 const Tensor &quat, const Volume *vol, const World *world,
-                                 const Projected *out) {
-        ctx->saved_data["vol"] = std::vector<int64_t>{vol->D, vol->H, vol->W};
+                                 const Tensor &quat, const Tensor &, const Volume *vol,
+                                 const World *world, const Projected *out) {
+        ctx->saved_data["vol"] =
+            std::vector<int64_t>{vol->D, vol->H, vol->W, pos.size(0), pos.get_device()};
         ctx->saved_data["world"] = std::vector<double>{world->wz, world->wy, world->wx,
                                                        world->cz, world->cy, world->cx};
         ctx->save_for_backward({pos, scale, quat, out->pos_radii});
@@ -123,14 +140,18 @@ struct Project : public torch::autograd::Function<Project> {
 
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         const auto saved = ctx->get_saved_variables();
-        const Tensor &pos = saved[0], &pos_radii = saved[3];
         const auto vol = ctx->saved_data["vol"].toIntVector();
         const auto w = ctx->saved_data["world"].toDoubleVector();
-        const int64_t n = pos.size(0);
-        const c10::DeviceGuard guard(pos.device());
+        const int64_t n = vol[3];
+        const at::Device dev = gpu(vol[4]);
+        const c10::DeviceGuard guard(dev);
+        const Tensor pos = unpacked(saved[0], at::kFloat, dev, n * 3, "pos3d");
+        const Tensor scale = unpacked(saved[1], at::kFloat, dev, n * 3, "scale3d");
+        const Tensor quat = unpacked(saved[2], at::kFloat, dev, n * 4, "quat");
+        const Tensor pos_radii = unpacked(saved[3], at::kFloat, dev, n * 4, "pos3d_radii");
         const auto given = [&](const Tensor &g, int64_t width, const char *what) {
             if (!g.defined()) return at::zeros({n, width}, pos_radii.options());
-            TORCH_CHECK(g.is_cuda() && g.scalar_type() == at::kFloat && g.numel() == n * width,
+            TORCH_CHECK(g.device() == dev && g.scalar_type() == at::kFloat && g.numel() == n * width,
                         what, ": expected ", n, " rows of ", width, " float32 values on the GPU");
             return g.contiguous();
         };
@@ -138,14 +159,14 @@ struct Project : public torch::autograd::Function<Project> {
         const Tensor dcn = given(grads[1], 6, "conics_grad_in");
         Tensor dpos = empty({n, 3}, pos, at::kFloat), dscale = empty({n, 3}, pos, at::kFloat);
         Tensor dquat = empty({n, 4}, pos, at::kFloat);
-        check(lib.gsv_project_bwd((int)n, ptr<float>(pos), ptr<float>(saved[1]),
-                                  ptr<float>(saved[2]), (int)vol[0], (int)vol[1], (int)vol[2],
+        check(lib.gsv_project_bwd((int)n, ptr<float>(pos), ptr<float>(scale),
+                                  ptr<float>(quat), (int)vol[0], (int)vol[1], (int)vol[2],
                                   (float)w[0], (float)w[1], (float)w[2], (float)w[3], (float)w[4],
                                   (float)w[5], ptr<float>(dpr), ptr<float>(dcn),
                                   ptr<float>(pos_radii), ptr<float>(dpos), ptr<float>(dscale),
                                   ptr<float>(dquat), stream_of(pos)),
               "project_bwd");
-        return {dpos, dscale, dquat, Tensor(), Tensor(), Tensor()};
+        return {dpos, dscale, dquat, Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -177,7 +198,7 @@ std::vector<Tensor> project(const Tensor &pos, const Tensor &scale, const Tensor
                               ptr<int32_t>(out.tile_min), ptr<int32_t>(out.tile_max),
                               ptr<int32_t>(out.hits), stream_of(pos)),
           "project_fwd");
-    return Project::apply(pos, scale, quat, &vol, &world, &out);
+    return Project::apply(pos, scale, quat, intens, &vol, &world, &out);
 }
 
 // ----------------------------------------------------------- voxelization --
@@ -188,20 +209,44 @@ struct Voxelized {
     int64_t count = -1;
 };
 
-// The backward of both nodes; sign and grad_loss are undefined without the loss.
-variable_list voxelize_backward(const Volume &vol, int64_t count, bool per_gaussian,
-                                const variable_list &saved, const Tensor &sign,
-                                const Tensor &grad_loss, const Tensor &grad_volume) {
-    const Tensor &pr = saved[0], &cn = saved[1], &intens = saved[2], &ids = saved[3];
-    const Tensor &bins = saved[4], &tile_min = saved[5], &tile_max = saved[6], &cum = saved[7];
-    const Tensor &tiles = saved[8], &live = saved[9];
-    const int n = (int)pr.size(0), C = (int)intens.size(1);
+// What a node keeps beside its tensors.
+struct Kept {
+    Volume vol;
+    int64_t count, cap, n, channels, device;
+    bool per_gaussian;
+
+    explicit Kept(const std::vector<int64_t> &m)
+        : vol{(int)m[0], (int)m[1], (int)m[2]}, count(m[3]), cap(m[4]), n(m[5]), channels(m[6]),
+          device(m[7]), per_gaussian(m[8] != 0) {}
+    int64_t voxels() const { return (int64_t)vol.D * vol.H * vol.W; }
+};
+
+// The backward of both nodes; grad_loss is undefined without the loss, whose
+// sign bytes are the last saved tensor.
+variable_list voxelize_backward(const Kept &k, const variable_list &saved, const Tensor &grad_loss,
+                                const Tensor &grad_volume) {
+    const Volume &vol = k.vol;
+    const int64_t count = k.count;
+    const int n = (int)k.n, C = (int)k.channels;
+    const at::Device dev = gpu(k.device);
+    const Tensor pr = unpacked(saved[0], at::kFloat, dev, k.n * 4, "pos3d_radii");
+    const Tensor cn = unpacked(saved[1], at::kFloat, dev, k.n * 6, "conics");
+    const Tensor intens = unpacked(saved[2], at::kFloat, dev, k.n * C, "intensities");
+    const Tensor ids = unpacked(saved[3], at::kInt, dev, k.cap, "gaussian_ids_sorted");
+    const Tensor bins = unpacked(saved[4], at::kInt, dev, vol.tiles() * 2, "tile_bins");
+    const Tensor tile_min = unpacked(saved[5], at::kInt, dev, k.n * 3, "tile_min");
+    const Tensor tile_max = unpacked(saved[6], at::kInt, dev, k.n * 3, "tile_max");
+    const Tensor cum = unpacked(saved[7], at::kInt, dev, k.n, "cum_tiles_hit");
+    const Tensor tiles = unpacked(saved[8], at::kInt, dev, k.cap, "tiles_sorted");
+    const Tensor live = unpacked(saved[9], at::kByte, dev, k.cap, "pair_live");
+    Tensor sign;
+    if (grad_loss.defined()) sign = unpacked(saved[10], at::kChar, dev, k.voxels() * C, "sign");
     Tensor vg;
     if (grad_volume.defined()) {
         vg = grad_volume.contiguous();
-        TORCH_CHECK(vg.is_cuda(), "vol_grad_in must be a CUDA tensor");
+        TORCH_CHECK(vg.device() == dev, "vol_grad_in must be a CUDA tensor on ", dev);
         TORCH_CHECK(vg.scalar_type() == at::kFloat, "vol_grad_in: expected scalar type float32");
-        TORCH_CHECK(vg.numel() == (int64_t)vol.D * vol.H * vol.W * C,
+        TORCH_CHECK(vg.numel() == k.voxels() * C,
                     "vol_grad_in must have D*H*W*channels elements");
     }
     Tensor dpos = empty({n, 4}, pr, at::kFloat), dconics = empty({n, 6}, pr, at::kFloat);
@@ -211,9 +256,9 @@ variable_list voxelize_backward(const Volume &vol, int64_t count, bool per_gauss
           "voxelize_bwd_workspace_bytes");
     const Tensor ws = workspace(bytes, pr);
     void *stream = stream_of(pr);
-    const int variant = per_gaussian ? 1 : 0;
+    const int variant = k.per_gaussian ? 1 : 0;
     if (sign.defined()) {
-        TORCH_CHECK(grad_loss.is_cuda() && grad_loss.scalar_type() == at::kFloat &&
+        TORCH_CHECK(grad_loss.device() == dev && grad_loss.scalar_type() == at::kFloat &&
                         grad_loss.numel() == 1,
                     "grad_loss must be one float32 value on the GPU");
         const Tensor gl = grad_loss.contiguous();
@@ -237,8 +282,10 @@ variable_list voxelize_backward(const Volume &vol, int64_t count, bool per_gauss
     return {dpos, dconics, dint};
 }
 
-variable_list zero_gradients(const variable_list &saved) {
-    return {at::zeros_like(saved[0]), at::zeros_like(saved[1]), at::zeros_like(saved[2])};
+variable_list zero_gradients(const Kept &k) {
+    const auto options = at::TensorOptions().device(gpu(k.device)).dtype(at::kFloat);
+    return {at::zeros({k.n, 4}, options), at::zeros({k.n, 6}, options),
+            at::zeros({k.n, k.channels}, options)};
 }
 
 variable_list saved_inputs(const Tensor &pr, const Tensor &cn, const Tensor &intens,
@@ -246,8 +293,11 @@ variable_list saved_inputs(const Tensor &pr, const Tensor &cn, const Tensor &int
     return {pr, cn, intens, v.ids, v.bins, v.tile_min, v.tile_max, v.cum, v.tiles, v.live};
 }
 
-void remember(AutogradContext *ctx, const Volume &vol, const Voxelized &v, bool per_gaussian) {
-    ctx->saved_data["vol"] = std::vector<int64_t>{vol.D, vol.H, vol.W, v.count, per_gaussian};
+void remember(AutogradContext *ctx, const Volume &vol, const Voxelized &v, const Tensor &intens,
+              bool per_gaussian) {
+    ctx->saved_data["kept"] = std::vector<int64_t>{
+        vol.D, vol.H, vol.W, v.count, v.ids.numel(), intens.size(0), intens.size(1),
+        intens.get_device(), per_gaussian};
     ctx->set_materialize_grads(false);
 }
 
@@ -255,29 +305,27 @@ struct Voxelize : public torch::autograd::Function<Voxelize> {
     static Tensor forward(AutogradContext *ctx, const Tensor &pr, const Tensor &cn,
                           const Tensor &intens, const Volume *vol, const Voxelized *v,
                           bool per_gaussian) {
-        remember(ctx, *vol, *v, per_gaussian);
+        remember(ctx, *vol, *v, intens, per_gaussian);
         ctx->save_for_backward(saved_inputs(pr, cn, intens, *v));
         return v->volume;
     }
 
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         const auto saved = ctx->get_saved_variables();
-        const auto m = ctx->saved_data["vol"].toIntVector();
-        const c10::DeviceGuard guard(saved[0].device());
-        variable_list g =
-            grads[0].defined()
-                ? voxelize_backward({(int)m[0], (int)m[1], (int)m[2]}, m[3], m[4] != 0, saved,
-                                    Tensor(), Tensor(), grads[0])
-                : zero_gradients(saved);
+        const Kept k(ctx->saved_data["kept"].toIntVector());
+        const c10::DeviceGuard guard(gpu(k.device));
+        variable_list g = grads[0].defined() ? voxelize_backward(k, saved, Tensor(), grads[0])
+                                             : zero_gradients(k);
         return {g[0], g[1], g[2], Tensor(), Tensor(), Tensor()};
     }
 };
 
 struct VoxelizeL1 : public torch::autograd::Function<VoxelizeL1> {
+    // The target gets no gradient, but makes the outputs require one.
     static variable_list forward(AutogradContext *ctx, const Tensor &pr, const Tensor &cn,
-                                 const Tensor &intens, const Volume *vol, const Voxelized *v,
-                                 bool per_gaussian) {
-        remember(ctx, *vol, *v, per_gaussian);
+                                 const Tensor &intens, const Tensor &, const Volume *vol,
+                                 const Voxelized *v, bool per_gaussian) {
+        remember(ctx, *vol, *v, intens, per_gaussian);
         auto saved = saved_inputs(pr, cn, intens, *v);
         saved.push_back(v->sign);
         ctx->save_for_backward(saved);
@@ -286,19 +334,19 @@ struct VoxelizeL1 : public torch::autograd::Function<VoxelizeL1> {
 
     static variable_list backward(AutogradContext *ctx, const variable_list &grads) {
         const auto saved = ctx->get_saved_variables();
-        const auto m = ctx->saved_data["vol"].toIntVector();
-        const c10::DeviceGuard guard(saved[0].device());
+        const Kept k(ctx->saved_data["kept"].toIntVector());
+        const c10::DeviceGuard guard(gpu(k.device));
         variable_list g;
         if (!grads[0].defined() && !grads[1].defined()) {
-            g = zero_gradients(saved);
+            g = zero_gradients(k);
         } else {
-            const Tensor gl = grads[0].defined()
-                                  ? grads[0]
-                                  : at::zeros({}, saved[0].options().dtype(at::kFloat));
-            g = voxelize_backward({(int)m[0], (int)m[1], (int)m[2]}, m[3], m[4] != 0, saved,
-                                  saved[10], gl, grads[1]);
+            const Tensor gl =
+                grads[0].defined()
+                    ? grads[0]
+                    : at::zeros({}, at::TensorOptions().device(gpu(k.device)).dtype(at::kFloat));
+            g = voxelize_backward(k, saved, gl, grads[1]);
         }
-        return {g[0], g[1], g[2], Tensor(), Tensor(), Tensor()};
+        return {g[0], g[1], g[2], Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -402,7 +450,7 @@ std::tuple<int64_t, std::vector<Tensor>> voxelize(
     Voxelized v;
     if (!voxelize_forward(pr, cn, intens, tile_min, tile_max, hits, t, vol, cap, slot, v))
         return {v.count, {}};
-    if (t.defined()) return {v.count, VoxelizeL1::apply(pr, cn, intens, &vol, &v, per_gaussian)};
+    if (t.defined()) return {v.count, VoxelizeL1::apply(pr, cn, intens, t, &vol, &v, per_gaussian)};
     return {v.count, {Voxelize::apply(pr, cn, intens, &vol, &v, per_gaussian)}};
 }
 

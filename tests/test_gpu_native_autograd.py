@@ -125,3 +125,50 @@ def test_hooks_streams_and_refusals(device):
         volume(inten.double())
     with pytest.raises(ValueError):
         o.optim_to_render(leaves[0][:0], *leaves[1:], cfg.vol, cfg.world, cfg.center)
+
+
+@pytest.mark.parametrize("change", ["cpu", "half", "shorter"])
+@pytest.mark.parametrize("node", ["project", "volume", "l1"])
+def test_saved_tensors_that_hooks_exchanged_are_refused(device, node, change):
+    """What the hooks hand back is checked on the host, before its address is used."""
+    from gs_voxelizer import optim_to_render as o, voxelize as v
+    leaves, cfg = _leaves(device)
+    target = torch.rand(cfg.vol + (1,), device=device)
+    _run(leaves, cfg, True, "volume", target)
+    unpack = {"cpu": lambda t: t.cpu(), "half": lambda t: t.half(),
+              "shorter": lambda t: t.flatten()[:-1]}[change]
+    hooks = torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack)
+    pr, cn, tmin, tmax, nt = o.optim_to_render(*(t.detach() for t in leaves), cfg.vol, cfg.world,
+                                               cfg.center)
+    args = (pr, cn, leaves[3], cfg.vol, tmin, tmax, nt)
+    with hooks:
+        if node == "project":
+            out = o.optim_to_render(*leaves, cfg.vol, cfg.world, cfg.center)[0]
+        elif node == "volume":
+            out = v.voxelize_gaussians(*args)
+        else:
+            out = v.voxelize_gaussians_l1_loss(*args, target)[0]
+    assert "CppNode" in out.grad_fn.name()
+    with pytest.raises(RuntimeError, match="values of scalar type"):
+        out.sum().backward()
+
+
+def test_what_makes_the_outputs_require_gradients(device):
+    """As with the classes: any argument does, also one that gets no gradient."""
+    from gs_voxelizer import optim_to_render as o, voxelize as v
+    leaves, cfg = _leaves(device)
+    target = torch.rand(cfg.vol + (1,), device=device)
+    _run(leaves, cfg, True, "volume", target)
+    pos, scale, quat, inten = (t.detach() for t in leaves)
+    for asks in (False, True):
+        pr, cn, tmin, tmax, nt = o.optim_to_render(pos, scale, quat,
+                                                   inten.clone().requires_grad_(asks), cfg.vol,
+                                                   cfg.world, cfg.center)
+        assert pr.requires_grad is asks and cn.requires_grad is asks
+        wanted = target.clone().requires_grad_(asks)
+        loss, vol = v.voxelize_gaussians_l1_loss(pr.detach(), cn.detach(), inten, cfg.vol, tmin,
+                                                 tmax, nt, wanted)
+        assert loss.requires_grad is asks and vol.requires_grad is asks
+        if asks:
+            loss.backward()
+            assert wanted.grad is None
