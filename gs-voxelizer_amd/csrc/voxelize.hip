@@ -1936,11 +1936,23 @@ __attribute__((amdgpu_waves_per_eu((C == 2 || C == 3) && kRows == 1 ? 2 : 1, 8))
 #pragma clang diagnostic pop
 
 // The pairs that k_vox_bwd left: those of the waves spanning more than K tiles,
-// in groups of K tiles after the first.  A fixed grid of kRestBlocks
-// workgroups; workgroup b reads the flags of the waves b, b + G, b + 2G, ...
-// (G = the grid size) 64 at a time, so the waves to process (many in a sparse
-// scene, none in most dense ones) spread over the whole grid.
-constexpr int kRestBlocks = 512;
+// in groups of K tiles after the first.  Workgroup b reads the flags of the
+// waves b, b + G, b + 2G, ... (G = the grid size) 64 at a time, so the waves to
+// process (many in a sparse scene, none in most dense ones) spread over the grid.
+//
+// The grid: a workgroup walks its flagged waves one after another, each a chain of
+// gathers and a row loop, so a scene that flags many (thin edge tiles, sparse
+// regions) needs more workgroups than one for every second SIMD; past ~8 a CU the
+// LDS of C > 2 leaves no room.  One for 8 waves of pairs keeps small scenes small.
+// us at 512 workgroups and by this rule: 44.7, 25.4 (157 x 203 x 181 / 120k / C =
+// 3), 227, 162 (256^3 / 500k clustered / C = 4), 10.3, 5.4 (512^3 / 1M), 4.7, 4.7
+// (256^3 / 200k), 4.5, 4.6 (128^3 / 50k); up to 4,096, one for 4 waves: 27.1 and
+// 165 in the first two.
+constexpr int64_t kRestMinBlocks = 512, kRestMaxBlocks = 2048, kRestWavesPerBlock = 8;
+
+unsigned rest_blocks(int64_t waves) {
+    return (unsigned)std::min(std::max(waves / kRestWavesPerBlock, kRestMinBlocks), kRestMaxBlocks);
+}
 
 template <int C, int K>
 __global__ __launch_bounds__(kWave) void k_vox_bwd_rest(BwdArgs a) {
@@ -2300,16 +2312,16 @@ int voxelize_bwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t
                                args);                                                               \
             if (int st = check_launch()) return st;                                                 \
             hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTilesVerySparse<CH>>),                     \
-                               dim3(kRestBlocks), block, 0, s, args);                               \
+                               dim3(rest_blocks(waves)), block, 0, s, args);                               \
         } else if (sparse) {                                                                        \
             hipLaunchKernelGGL((k_vox_bwd<CH, kStageTilesSparse<CH>, 1>), grid, block, 0, s, args);   \
             if (int st = check_launch()) return st;                                                 \
-            hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTilesSparse<CH>>), dim3(kRestBlocks),     \
+            hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTilesSparse<CH>>), dim3(rest_blocks(waves)),     \
                                block, 0, s, args);                                                  \
         } else {                                                                                    \
             hipLaunchKernelGGL((k_vox_bwd<CH, kStageTiles<CH>, 1>), grid, block, 0, s, args);         \
             if (int st = check_launch()) return st;                                                 \
-            hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTiles<CH>>), dim3(kRestBlocks), block, 0, \
+            hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTiles<CH>>), dim3(rest_blocks(waves)), block, 0, \
                                s, args);                                                            \
         }                                                                                           \
     }                                                                                               \

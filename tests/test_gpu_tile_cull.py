@@ -290,7 +290,7 @@ def test_small_scene_backward_matches_the_rest_pass(device, set_chains, channels
     assert 0 < I < 2048 * 64
     g = torch.randn(vol + (channels,), device=device)
     grads = []
-    for cap in (I, 2049 * 64):
+    for cap in (I, 2049 * 64, 6000 * 64, 20000 * 64):  # the last two: larger rest grids
         ids, bins, tiles = _C.bin_and_sort_gaussians_device_count(n, cap, total, tmin, tmax, cum,
                                                                   vol, return_tiles=True)
         live = torch.empty(cap, device=device, dtype=torch.uint8)
@@ -298,5 +298,6 @@ def test_small_scene_backward_matches_the_rest_pass(device, set_chains, channels
         grads.append(_C.voxelize_backward_per_gaussian(
             vol, ids, bins, pr, cn, work.intensities, g, tmin, tmax, cum, tiles_sorted=tiles,
             count_dev=total, pair_live=live))
-    for a, b in zip(*grads):
-        assert torch.equal(a, b)
+    for other in grads[1:]:
+        for a, b in zip(grads[0], other):
+            assert torch.equal(a, b)
