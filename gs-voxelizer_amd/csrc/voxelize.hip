@@ -296,7 +296,7 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-// At least six waves per SIMD at C = 1 (66 VGPRs, no spills, so seven; five and
+// At least six waves per SIMD at C = 1 (68 VGPRs, no spills, so seven; five and
 // eight, at 64, measured within 1 % of it); more channels would spill at six.
 //
 // S waves per tile (fwd_split chooses S), each walking an equal share of the
@@ -367,21 +367,15 @@ __attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, 8))) void k_vox_fwd(
                 // centred offsets: delta = c - p', p' = local index - 3.5
                 const float cx = p.x - (float)tg.x0 - 4.0f;
                 const float cy = p.y - (float)tg.y0 - 4.0f, cz = p.z - (float)tg.z0 - 4.0f;
-                // Q c and c^T Q c in binary64: the culling test and the rows' terms
-                // about the tile centre are both formed from them (a batch's set-up
-                // is ~13 % of the kernel's VALU time, most of it binary64 at 4 cycles
-                // an instruction; formed apart, with the box test, k_vox_fwd took
-                // 173 us at 256^3 / 200k instead of 167, 1.35 ms at 512^3 / 1M
-                // instead of 1.29)
-                double nx = 0.0, ny = 0.0, nz = 0.0, m = 0.0;
-                if (live) {
+                // the culling test from the conic itself, in binary64
+                if (live && gt.bounded &&
+                    positive_definite(c01.x, c01.y, c23.x, c23.y, c45.x, c45.y)) {
                     const double X = cx, Y = cy, Z = cz, b = c01.y, c = c23.x, e = c45.x;
-                    nx = fma((double)c01.x, X, fma(b, Y, c * Z));
-                    ny = fma(b, X, fma((double)c23.y, Y, e * Z));
-                    nz = fma(c, X, fma(e, Y, (double)c45.y * Z));
-                    m = fma(X, nx, fma(Y, ny, Z * nz));
-                    if (gt.bounded && positive_definite(c01.x, c01.y, c23.x, c23.y, c45.x, c45.y))
-                        live = !misses_tile((float)m, (float)(fabs(nx) + fabs(ny) + fabs(nz)), gt.t2);
+                    const double nx = fma((double)c01.x, X, fma(b, Y, c * Z));
+                    const double ny = fma(b, X, fma((double)c23.y, Y, e * Z));
+                    const double nz = fma(c, X, fma(e, Y, (double)c45.y * Z));
+                    const double m = fma(X, nx, fma(Y, ny, Z * nz));
+                    live = !misses_tile((float)m, (float)(fabs(nx) + fabs(ny) + fabs(nz)), gt.t2);
                 }
                 if (live) {
                     // the gate-free rows expand the form about the tile centre, whose
@@ -402,14 +396,25 @@ __attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, 8))) void k_vox_fwd(
                         //   T1 = t1 - B py - C pz,
                         //   T0 = t0 + ty py + tz pz + D py^2 + E py pz + F pz^2,
                         // t0 = the form at the tile centre, ty/tz its y/z slopes there.
-                        // Formed in binary64 from the conic itself and rounded once.
+                        // Formed in binary64 and rounded once, from the same rounded
+                        // coefficients A2 .. F as the rows' other terms: their error
+                        // is then that of a slightly different conic, small where the
+                        // form is small.  From the conic itself (one set of products
+                        // for the culling test and these: k_vox_fwd 209 instead of 212
+                        // us at 256^3 / 200k, 1.40 instead of 1.42 ms at 512^3 / 1M)
+                        // the coefficients' rounding stays at the Gaussian's centre,
+                        // times the tile's size: 15 % more error at axes of 1/60 voxel.
                         // (t1, -B, -C, t0 | ty, tz, D, E | F, Q0, Q1, Q2 | Q3, I*2^-off ...),
                         // Q_k = A2 * uc_k^2 + off for the four |uc| = 0.5, 1.5, 2.5, 3.5
-                        constexpr double kL = 1.4426950408889634074;  // log2(e)
-                        const double t1 = -kL * nx, t0 = (-0.5 * kL) * m;
+                        const double X = cx, Y = cy, Z = cz;
+                        const double a2 = A2, bb = q1.x, cc = q1.y, dd = q1.z, ee = q1.w, ff = F;
+                        const double t1 = 2.0 * a2 * X + bb * Y + cc * Z;
                         rec[0] = (float)t1;
                         rec[1] = -q1.x; rec[2] = -q1.y;
-                        const double ty = kL * ny, tz = kL * nz;
+                        const double t0 = X * (a2 * X + bb * Y + cc * Z) + Y * (dd * Y + ee * Z) +
+                                          ff * Z * Z;
+                        const double ty = -(bb * X + 2.0 * dd * Y + ee * Z);
+                        const double tz = -(cc * X + ee * Y + 2.0 * ff * Z);
                         rec[6] = q1.z; rec[7] = q1.w;
                         rec[8] = F;
                         // Chained rows (the first two loops below) split s(u) into

@@ -363,3 +363,42 @@ def test_forward_waves_sharing_a_tile(device, vol, n, channels):
     pad = torch.cat([p["ids"], torch.zeros(3 * p["I"] + 64, device=device, dtype=torch.int32)])
     again = _C.voxelize_forward(vol, pad, p["bins"], p["pr"], p["cn"], p["w"].intensities)
     assert torch.equal(out, again)
+
+
+@pytest.mark.parametrize("channels", [1, 3])
+@pytest.mark.parametrize("q", [89.21875, 1001.078125])
+def test_forward_peak_does_not_depend_on_the_place_in_the_tile(device, q, channels):
+    """Thin Gaussians at the corners of their tiles, one to a tile: the rows expand
+    the form about the tile's centre with coefficients fl(-log2(e)/2 * q), and these
+    conics are ones that such a coefficient misses by 5e-8 to 7e-8 of itself.  All
+    terms have to come from that coefficient; a constant term formed from q leaves
+    the coefficient's error times the corner's 36.75 square voxels at the Gaussian's
+    centre (1.7e-4 and 1.5e-3 in the exponent).  The bound on the mean error of the
+    exponent: the rounding of the one term that all the tiles share (the row end's
+    A2 * 3.5^2 + offset, the offset above -127), and 5 standard deviations of the
+    mean of at most 14 roundings of partial sums below 4 * A2 * 36.75."""
+    import gs_voxelizer.cuda as _C
+    edge, u = 256, 2.0 ** -24
+    Tx = edge // 8
+    n = Tx ** 3
+    g = torch.Generator().manual_seed(int(q))
+    t = torch.arange(n)
+    origin = 8.0 * torch.stack([t % Tx, t // Tx % Tx, t // Tx ** 2], 1).double()
+    voxel = origin + 7.0 * torch.randint(0, 2, (n, 3), generator=g) + 0.5
+    centre = (voxel + 0.02 * (torch.rand((n, 3), generator=g).double() - 0.5)).float()
+    pr = torch.cat([centre, torch.ones(n, 1)], 1).to(device)
+    conics = torch.tensor([q, 0.0, 0.0, q, 0.0, q]).repeat(n, 1).to(device)
+    ids = t.to(device, torch.int32)
+    bins = torch.stack([ids, ids + 1], 1)
+    out = _C.voxelize_forward((edge,) * 3, ids, bins, pr, conics,
+                              torch.ones(n, channels, device=device))
+    x, y, z = (voxel - 0.5).long().unbind(1)
+    got = out.cpu()[z, y, x].double()
+    d2 = ((centre.double() - voxel) ** 2).sum(1)
+    a2 = 0.5 * np.log2(np.e) * q
+    shared = u * (a2 * 12.25 + 127.0)
+    spread = u * 4.0 * a2 * 36.75 * np.sqrt(14.0 / 3.0)
+    for c in range(channels):
+        error = torch.log2(got[:, c]) + d2 * a2
+        assert abs(float(error.mean())) <= shared + 5.0 * spread / np.sqrt(n)
+        assert float(error.abs().max()) <= 14.0 * u * 4.0 * a2 * 36.75
