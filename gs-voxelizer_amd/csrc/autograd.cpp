@@ -350,17 +350,18 @@ struct VoxelizeL1 : public torch::autograd::Function<VoxelizeL1> {
     }
 };
 
-// The pair count that the prefix-sum kernel writes into pinned memory; -1 after
-// too many reads (the caller then takes the path that synchronises).
-int64_t await_count(const volatile int64_t *host) {
-    for (int64_t k = 0; k < ((int64_t)1 << 31); ++k) {
-        const int64_t v = *host;
-        if (v >= 0) {
-            std::atomic_thread_fence(std::memory_order_acquire);
-            return v;
-        }
+// The pair count that the prefix-sum kernel writes into pinned memory, read up to
+// `reads` times and then once more behind the stream's work (a long queue ahead
+// of this forward); negative when even that work left none.
+int64_t await_count(const volatile int64_t *host, int64_t reads, const at::Device &dev) {
+    int64_t v = *host;
+    for (int64_t k = 1; v < 0 && k < reads; ++k) v = *host;
+    if (v < 0) {
+        c10::hip::getCurrentHIPStream(dev.index()).synchronize();
+        v = *host;
     }
-    return -1;
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return v;
 }
 
 // Prefix sum, binning and forward at the capacity (target: the fused L1 step).
@@ -368,7 +369,7 @@ int64_t await_count(const volatile int64_t *host) {
 bool voxelize_forward(const Tensor &pr, const Tensor &cn, const Tensor &intens,
                       const Tensor &tile_min, const Tensor &tile_max, const Tensor &hits,
                       const Tensor &target, const Volume &vol, int64_t cap, const Tensor &slot,
-                      Voxelized &v) {
+                      int64_t reads, Voxelized &v) {
     const int64_t n = pr.size(0);
     const int C = (int)intens.size(1);
     int64_t *host = static_cast<int64_t *>(slot.data_ptr());
@@ -411,7 +412,7 @@ bool voxelize_forward(const Tensor &pr, const Tensor &cn, const Tensor &intens,
                                    ptr<uint8_t>(v.live), stream),
               "voxelize_fwd");
     }
-    v.count = await_count(host);
+    v.count = await_count(host, reads, pr.device());
     return v.count >= 1 && v.count <= cap;
 }
 
@@ -421,7 +422,7 @@ bool voxelize_forward(const Tensor &pr, const Tensor &cn, const Tensor &intens,
 std::tuple<int64_t, std::vector<Tensor>> voxelize(
     const Tensor &pr, const Tensor &cn, const Tensor &intens, const Tensor &tile_min,
     const Tensor &tile_max, const Tensor &hits, const c10::optional<Tensor> &target, int64_t D,
-    int64_t H, int64_t W, bool per_gaussian, int64_t cap, const Tensor &slot) {
+    int64_t H, int64_t W, bool per_gaussian, int64_t cap, const Tensor &slot, int64_t reads) {
     const std::tuple<int64_t, std::vector<Tensor>> none{-1, {}};
     if (!pr.defined() || !pr.is_cuda() || pr.dim() != 2 || !fits(D, H, W) || cap < 1) return none;
     const int64_t n = pr.size(0);
@@ -448,7 +449,8 @@ std::tuple<int64_t, std::vector<Tensor>> voxelize(
     }
     const c10::DeviceGuard guard(dev);
     Voxelized v;
-    if (!voxelize_forward(pr, cn, intens, tile_min, tile_max, hits, t, vol, cap, slot, v))
+    if (!voxelize_forward(pr, cn, intens, tile_min, tile_max, hits, t, vol, cap, slot,
+                          reads, v))
         return {v.count, {}};
     if (t.defined()) return {v.count, VoxelizeL1::apply(pr, cn, intens, t, &vol, &v, per_gaussian)};
     return {v.count, {Voxelize::apply(pr, cn, intens, &vol, &v, per_gaussian)}};

@@ -41,6 +41,7 @@ def _speculate() -> bool:
 
 
 _SPIN_READS = 1 << 21  # reads of the pinned count before falling back to a device sync
+_NATIVE_SPIN_READS = 1 << 28  # and in the native node, before it waits for the stream
 
 
 def _count_slot(dev: torch.device) -> Tensor:
@@ -160,7 +161,7 @@ def _native_voxelize(pos3d_radii, conics, intensities, vol_size_voxel, tile_min,
         return None
     D, H, W = (int(v) for v in vol_size_voxel)
     count, out = _native.voxelize(*tensors, target, D, H, W, bool(use_per_gaussian_backward), cap,
-                                  _count_slot(dev))
+                                  _count_slot(dev), _NATIVE_SPIN_READS)
     if (count > cap and count <= _INT32_MAX) or (out and count < cap // 4):
         _capacity[dev.index] = _grow(count)
     return out

@@ -172,3 +172,21 @@ def test_what_makes_the_outputs_require_gradients(device):
         if asks:
             loss.backward()
             assert wanted.grad is None
+
+
+@pytest.mark.parametrize("reads", [0, 1])
+@pytest.mark.parametrize("use", ["volume", "l1"])
+def test_a_count_that_is_late_is_waited_for(device, monkeypatch, use, reads):
+    """Out of reads of the pinned count, the native node waits for its stream and
+    keeps what it launched; the class does not launch the forward again."""
+    from gs_voxelizer import voxelize as v
+    leaves, cfg = _leaves(device)
+    target = torch.rand(cfg.vol + (1,), device=device)
+    _run(leaves, cfg, True, use, target)
+    ref = _run(leaves, cfg, True, use, target)
+
+    def entered(*args):
+        raise AssertionError("the class launched a forward")
+    monkeypatch.setattr(v, "_bin_and_forward", entered)
+    monkeypatch.setattr(v, "_NATIVE_SPIN_READS", reads)
+    _same(_run(leaves, cfg, False, use, target), ref)
