@@ -17,6 +17,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <atomic>
+#include <iterator>
 #include <map>
 #include <string>
 #include <tuple>
@@ -221,8 +222,7 @@ struct Kept {
     int64_t voxels() const { return (int64_t)vol.D * vol.H * vol.W; }
 };
 
-// The backward of both nodes; grad_loss is undefined without the loss, whose
-// sign bytes are the last saved tensor.
+// The backward of both nodes; grad_loss is undefined without the loss.
 variable_list voxelize_backward(const Kept &k, const variable_list &saved, const Tensor &grad_loss,
                                 const Tensor &grad_volume) {
     const Volume &vol = k.vol;
@@ -232,15 +232,16 @@ variable_list voxelize_backward(const Kept &k, const variable_list &saved, const
     const Tensor pr = unpacked(saved[0], at::kFloat, dev, k.n * 4, "pos3d_radii");
     const Tensor cn = unpacked(saved[1], at::kFloat, dev, k.n * 6, "conics");
     const Tensor intens = unpacked(saved[2], at::kFloat, dev, k.n * C, "intensities");
-    const Tensor ids = unpacked(saved[3], at::kInt, dev, k.cap, "gaussian_ids_sorted");
+    const Tensor ids = unpacked(saved[3], at::kInt, dev, count, "gaussian_ids_sorted");
     const Tensor bins = unpacked(saved[4], at::kInt, dev, vol.tiles() * 2, "tile_bins");
-    const Tensor tile_min = unpacked(saved[5], at::kInt, dev, k.n * 3, "tile_min");
-    const Tensor tile_max = unpacked(saved[6], at::kInt, dev, k.n * 3, "tile_max");
-    const Tensor cum = unpacked(saved[7], at::kInt, dev, k.n, "cum_tiles_hit");
-    const Tensor tiles = unpacked(saved[8], at::kInt, dev, k.cap, "tiles_sorted");
-    const Tensor live = unpacked(saved[9], at::kByte, dev, k.cap, "pair_live");
+    size_t next = 5;
     Tensor sign;
-    if (grad_loss.defined()) sign = unpacked(saved[10], at::kChar, dev, k.voxels() * C, "sign");
+    if (grad_loss.defined()) sign = unpacked(saved[next++], at::kChar, dev, k.voxels() * C, "sign");
+    const Tensor tile_min = unpacked(saved[next++], at::kInt, dev, k.n * 3, "tile_min");
+    const Tensor tile_max = unpacked(saved[next++], at::kInt, dev, k.n * 3, "tile_max");
+    const Tensor cum = unpacked(saved[next++], at::kInt, dev, k.n, "cum_tiles_hit");
+    const Tensor tiles = unpacked(saved[next++], at::kInt, dev, count, "tiles_sorted");
+    const Tensor live = unpacked(saved[next++], at::kByte, dev, k.cap, "pair_live");
     Tensor vg;
     if (grad_volume.defined()) {
         vg = grad_volume.contiguous();
@@ -288,15 +289,21 @@ variable_list zero_gradients(const Kept &k) {
             at::zeros({k.n, k.channels}, options)};
 }
 
-variable_list saved_inputs(const Tensor &pr, const Tensor &cn, const Tensor &intens,
-                           const Voxelized &v) {
-    return {pr, cn, intens, v.ids, v.bins, v.tile_min, v.tile_max, v.cum, v.tiles, v.live};
+// The tensors, shapes and order that the classes save: a checkpointed forward on
+// one route may be computed again on the other.
+variable_list saved_tensors(const Tensor &pr, const Tensor &cn, const Tensor &intens,
+                            const Voxelized &v) {
+    variable_list saved{pr, cn, intens, v.ids.narrow(0, 0, v.count), v.bins};
+    if (v.sign.defined()) saved.push_back(v.sign);
+    const Tensor rest[] = {v.tile_min, v.tile_max, v.cum, v.tiles.narrow(0, 0, v.count), v.live};
+    saved.insert(saved.end(), std::begin(rest), std::end(rest));
+    return saved;
 }
 
 void remember(AutogradContext *ctx, const Volume &vol, const Voxelized &v, const Tensor &intens,
               bool per_gaussian) {
     ctx->saved_data["kept"] = std::vector<int64_t>{
-        vol.D, vol.H, vol.W, v.count, v.ids.numel(), intens.size(0), intens.size(1),
+        vol.D, vol.H, vol.W, v.count, v.live.numel(), intens.size(0), intens.size(1),
         intens.get_device(), per_gaussian};
     ctx->set_materialize_grads(false);
 }
@@ -306,7 +313,7 @@ struct Voxelize : public torch::autograd::Function<Voxelize> {
                           const Tensor &intens, const Volume *vol, const Voxelized *v,
                           bool per_gaussian) {
         remember(ctx, *vol, *v, intens, per_gaussian);
-        ctx->save_for_backward(saved_inputs(pr, cn, intens, *v));
+        ctx->save_for_backward(saved_tensors(pr, cn, intens, *v));
         return v->volume;
     }
 
@@ -326,9 +333,7 @@ struct VoxelizeL1 : public torch::autograd::Function<VoxelizeL1> {
                                  const Tensor &intens, const Tensor &, const Volume *vol,
                                  const Voxelized *v, bool per_gaussian) {
         remember(ctx, *vol, *v, intens, per_gaussian);
-        auto saved = saved_inputs(pr, cn, intens, *v);
-        saved.push_back(v->sign);
-        ctx->save_for_backward(saved);
+        ctx->save_for_backward(saved_tensors(pr, cn, intens, *v));
         return {v->loss, v->volume};
     }
 

@@ -190,3 +190,40 @@ def test_a_count_that_is_late_is_waited_for(device, monkeypatch, use, reads):
     monkeypatch.setattr(v, "_bin_and_forward", entered)
     monkeypatch.setattr(v, "_NATIVE_SPIN_READS", reads)
     _same(_run(leaves, cfg, False, use, target), ref)
+
+
+class _Watching(torch.overrides.TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("use", ["volume", "l1"])
+@pytest.mark.parametrize("empty", [False, True])
+def test_checkpoint_whose_recomputation_takes_the_other_route(device, use, empty):
+    """A checkpointed step runs its forward under a function mode (the classes) and
+    is computed again outside it (the native nodes): both keep the same tensors in
+    the same order, so the recomputation fits."""
+    from gs_voxelizer import optim_to_render as o, voxelize as v
+    from torch.utils.checkpoint import checkpoint
+    leaves, cfg = _leaves(device)
+    target = torch.rand(cfg.vol + (1,), device=device)
+    if empty:
+        with torch.no_grad():
+            leaves[0] += 50.0
+        _run(leaves, cfg, True, use, target)
+    _run(leaves, cfg, True, use, target)
+    ref = _run(leaves, cfg, True, use, target)
+
+    def step(*leaves):
+        pr, cn, tmin, tmax, nt = o.optim_to_render(*leaves, cfg.vol, cfg.world, cfg.center)
+        args = (pr, cn, leaves[3], cfg.vol, tmin, tmax, nt)
+        if use == "l1":
+            return v.voxelize_gaussians_l1_loss(*args, target)[0]
+        return F.mse_loss(v.voxelize_gaussians(*args), target)
+
+    for t in leaves:
+        t.grad = None
+    with _Watching():
+        loss = checkpoint(step, *leaves, use_reentrant=False)
+    loss.backward()
+    _same([loss] + [t.grad for t in leaves], ref[6:])
