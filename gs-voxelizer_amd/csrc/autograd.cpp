@@ -293,6 +293,10 @@ variable_list zero_gradients(const Kept &k) {
 // one route may be computed again on the other.
 variable_list saved_tensors(const Tensor &pr, const Tensor &cn, const Tensor &intens,
                             const Voxelized &v) {
+    if (v.count == 0) {
+        if (v.sign.defined()) return {pr, cn, intens, empty({0}, pr, at::kInt), v.bins, v.sign};
+        return {pr, cn, intens, empty({0, 1}, pr, at::kInt), empty({0, 3}, pr, at::kInt)};
+    }
     variable_list saved{pr, cn, intens, v.ids.narrow(0, 0, v.count), v.bins};
     if (v.sign.defined()) saved.push_back(v.sign);
     const Tensor rest[] = {v.tile_min, v.tile_max, v.cum, v.tiles.narrow(0, 0, v.count), v.live};
@@ -321,8 +325,9 @@ struct Voxelize : public torch::autograd::Function<Voxelize> {
         const auto saved = ctx->get_saved_variables();
         const Kept k(ctx->saved_data["kept"].toIntVector());
         const c10::DeviceGuard guard(gpu(k.device));
-        variable_list g = grads[0].defined() ? voxelize_backward(k, saved, Tensor(), grads[0])
-                                             : zero_gradients(k);
+        variable_list g = k.count > 0 && grads[0].defined()
+                              ? voxelize_backward(k, saved, Tensor(), grads[0])
+                              : zero_gradients(k);
         return {g[0], g[1], g[2], Tensor(), Tensor(), Tensor()};
     }
 };
@@ -342,7 +347,7 @@ struct VoxelizeL1 : public torch::autograd::Function<VoxelizeL1> {
         const Kept k(ctx->saved_data["kept"].toIntVector());
         const c10::DeviceGuard guard(gpu(k.device));
         variable_list g;
-        if (!grads[0].defined() && !grads[1].defined()) {
+        if (k.count < 1 || (!grads[0].defined() && !grads[1].defined())) {
             g = zero_gradients(k);
         } else {
             const Tensor gl =
@@ -418,12 +423,13 @@ bool voxelize_forward(const Tensor &pr, const Tensor &cn, const Tensor &intens,
               "voxelize_fwd");
     }
     v.count = await_count(host, reads, pr.device());
-    return v.count >= 1 && v.count <= cap;
+    return v.count >= 0 && v.count <= cap;
 }
 
 // (count, outputs): the volume, or (loss, volume) with a target.  No outputs
-// for a call that the Python class takes: inputs other than the plain ones, no
-// pairs, or more than the capacity holds.
+// for a call that the Python class takes: inputs other than the plain ones, or
+// more pairs than the capacity holds.  Without pairs every tile's range is empty:
+// the volume is zero, and the gradients are.
 std::tuple<int64_t, std::vector<Tensor>> voxelize(
     const Tensor &pr, const Tensor &cn, const Tensor &intens, const Tensor &tile_min,
     const Tensor &tile_max, const Tensor &hits, const c10::optional<Tensor> &target, int64_t D,

@@ -148,8 +148,8 @@ def _native_voxelize(pos3d_radii, conics, intensities, vol_size_voxel, tile_min,
     """The plain steady-state call through the native nodes (the same launches at
     the recorded capacity, the same count check): [volume], or [loss, volume]
     with a target.  None where the Python class has to do it: the first call on
-    the device, GSV_SYNC_COUNT=1, graph capture, inputs that are not plain, no
-    pairs, or more than the capacity holds (which is raised here first)."""
+    the device, GSV_SYNC_COUNT=1, graph capture, inputs that are not plain, or
+    more pairs than the capacity holds (which is raised here first)."""
     tensors = (pos3d_radii, conics, intensities, tile_min, tile_max, num_tiles_hit)
     if not _native.plain(*(tensors if target is None else tensors + (target,))):
         return None

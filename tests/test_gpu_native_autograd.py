@@ -227,3 +227,26 @@ def test_checkpoint_whose_recomputation_takes_the_other_route(device, use, empty
         loss = checkpoint(step, *leaves, use_reentrant=False)
     loss.backward()
     _same([loss] + [t.grad for t in leaves], ref[6:])
+
+
+@pytest.mark.parametrize("use", ["volume", "l1", "l1_volume_only", "l1_both"])
+def test_an_empty_scene_takes_one_forward(device, monkeypatch, use):
+    """No pairs: the native node's own launches give the zero volume (and the loss
+    against it); the class does not launch them again."""
+    from gs_voxelizer import voxelize as v
+    leaves, cfg = _leaves(device)
+    target = torch.rand(cfg.vol + (1,), device=device)
+    _run(leaves, cfg, True, use, target)  # records a capacity
+    with torch.no_grad():
+        leaves[0] += 50.0
+    cap = v._capacity[device.index or 0]
+    ref = _run(leaves, cfg, True, use, target)
+    v._capacity[device.index or 0] = cap
+
+    def entered(*args):
+        raise AssertionError("the class launched a forward")
+    monkeypatch.setattr(v, "_bin_and_forward", entered)
+    got = _run(leaves, cfg, False, use, target)
+    assert "CppNode" in got[5].grad_fn.name()
+    _same(got, ref)
+    assert v._capacity[device.index or 0] == v._grow(0)
