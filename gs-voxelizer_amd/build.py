@@ -5,7 +5,9 @@ hipcc compiles every ``csrc/*.hip`` for ``--offload-arch=gfx950`` and links one
 C-ABI shared library next to the Python package, where ``gs_voxelizer._lib``
 loads it.  No torch headers are involved, so the library is independent of the
 torch build's C++ ABI.  csrc/autograd.cpp (host code, g++) is the part that does
-use them: a Python extension module, gs_voxelizer/_autograd.so.
+use them: a Python extension module, gs_voxelizer/_autograd.so.  Where it cannot
+be built (no torch headers, no g++) the library is built all the same, and
+gs_voxelizer runs its Python autograd classes.
 """
 import os
 import shutil
@@ -70,9 +72,36 @@ def autograd_command(out):
                "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"])
 
 
+def _start_autograd(out, verbose):
+    """The running g++ of the autograd module, or the reason why there is none."""
+    try:
+        cmd = autograd_command(out)
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        return subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    except (ImportError, AttributeError, OSError) as e:
+        return f"{type(e).__name__}: {e}"
+
+
+def _install_autograd(started, out, verbose):
+    """Puts the autograd module in place; without one an older module goes too."""
+    if not isinstance(started, str):
+        log = started.communicate()[0]
+        if started.returncode == 0:
+            if verbose and log.strip():
+                print(log, flush=True)
+            os.replace(out, AUTOGRAD)
+            return
+        started = f"g++ ({started.returncode}):\n{log}"
+    if os.path.exists(AUTOGRAD):
+        os.remove(AUTOGRAD)
+    print(f"the native autograd nodes were not built: {started}", file=sys.stderr, flush=True)
+
+
 def build(verbose=False):
     """Compile the library and the autograd module; returns the library's path.
-    Always recompiles.
+    Always recompiles.  Raises where the library cannot be built; without the
+    autograd module it says why on stderr.
 
     Each source is compiled to an object in its own hipcc process (they run
     concurrently; every translation unit is self-contained), then one link
@@ -81,11 +110,7 @@ def build(verbose=False):
     flags = [f for f in HIPCC_FLAGS if f != "-shared"]
     with tempfile.TemporaryDirectory(dir=os.path.dirname(OUT)) as tmpdir:
         procs, tmp_autograd = [], os.path.join(tmpdir, "_autograd.so")
-        cmd = autograd_command(tmp_autograd)
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        procs.append(("autograd.cpp", None, subprocess.Popen(
-            cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+        autograd = _start_autograd(tmp_autograd, verbose)
         for s in SOURCES:
             obj = os.path.join(tmpdir, os.path.splitext(s)[0] + ".o")
             cmd = [hipcc()] + flags + SOURCE_FLAGS.get(s, []) + ["-c", os.path.join(CSRC, s), "-o", obj]
@@ -101,10 +126,11 @@ def build(verbose=False):
                 failed.append(f"{s} ({pr.returncode}):\n{log}")
             elif verbose and log.strip():
                 print(log, flush=True)
-            if obj:
-                objs.append(obj)
+            objs.append(obj)
         if failed:
-            raise RuntimeError("build failed: " + "\n".join(failed))
+            if not isinstance(autograd, str):
+                autograd.communicate()
+            raise RuntimeError("hipcc failed: " + "\n".join(failed))
         tmp = os.path.join(tmpdir, "libgsvox.so")
         cmd = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC"] + objs + ["-o", tmp]
         if verbose:
@@ -113,7 +139,7 @@ def build(verbose=False):
         if res.returncode != 0:
             raise RuntimeError(f"hipcc link failed ({res.returncode}):\n{_clean(res.stdout + res.stderr)}")
         os.replace(tmp, OUT)
-        os.replace(tmp_autograd, AUTOGRAD)
+        _install_autograd(autograd, tmp_autograd, verbose)
     return OUT
 
 
