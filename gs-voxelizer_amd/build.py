@@ -66,7 +66,8 @@ def autograd_command(out):
                sysconfig.get_paths()["include"]]
     return ([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
              "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_autograd",
-             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+             f'-DGSV_TORCH_VERSION="{torch.__version__}"']
             + ["-isystem" + d for d in include]
             + [os.path.join(CSRC, "autograd.cpp"), "-o", out, "-L" + os.path.join(base, "lib"),
                "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"])

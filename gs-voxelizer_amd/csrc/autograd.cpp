@@ -470,6 +470,7 @@ std::tuple<int64_t, std::vector<Tensor>> voxelize(
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    m.attr("torch_version") = GSV_TORCH_VERSION;  // the torch it was compiled against
     m.def("bind", &bind);
     m.def("project", &project, py::call_guard<py::gil_scoped_release>());
     m.def("voxelize", &voxelize, py::call_guard<py::gil_scoped_release>());

@@ -1,0 +1,42 @@
+"""The native autograd nodes are an addition to the Python classes: the package
+imports without them, or with a module of another torch, and says so once."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "gs-voxelizer_amd")
+
+MISSING = """
+import sys
+sys.modules["gs_voxelizer._autograd"] = None  # import raises ModuleNotFoundError
+"""
+OTHER_TORCH = """
+import sys, types
+m = types.ModuleType("gs_voxelizer._autograd")
+m.torch_version = "1.0.0"
+sys.modules["gs_voxelizer._autograd"] = m
+"""
+
+
+@pytest.mark.parametrize("before,why", [(MISSING, "_autograd"), (OTHER_TORCH, "torch 1.0.0")],
+                         ids=["missing", "other_torch"])
+def test_the_package_imports_without_the_nodes(before, why):
+    code = before + """
+import torch
+import gs_voxelizer.optim_to_render as o, gs_voxelizer.voxelize, gs_voxelizer.graph
+from gs_voxelizer import _native
+assert not _native.available and not _native.plain(torch.zeros(1))
+z = torch.zeros((0, 3))
+try:
+    o.optim_to_render(z, z, torch.zeros((0, 4)), torch.zeros((0, 1)), (8, 8, 8), (1.0, 1.0, 1.0),
+                      (0.5, 0.5, 0.5))
+except ValueError as e:
+    print(e)
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
+                       env=dict(os.environ, PYTHONPATH=PKG))
+    assert r.returncode == 0, r.stderr
+    assert "Invalid shape" in r.stdout
+    assert r.stderr.count("RuntimeWarning: gs_voxelizer: no native") == 1 and why in r.stderr
