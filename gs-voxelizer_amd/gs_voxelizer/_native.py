@@ -3,7 +3,8 @@
 Plain calls of ``optim_to_render`` and ``voxelize_gaussians`` (ordinary tensors,
 no transform or mode active) go to ``project`` and ``voxelize``, which return
 nothing for a call they do not take; the Python autograd classes then do it, and
-raise its errors.  Without a module built for this torch the classes do all calls
+raise its errors.  Without a module built for this torch, or in a torch that no
+longer has one of the private names that `plain` asks, the classes do all calls
 (same kernels and results, more host time), after a warning.
 """
 import ctypes
@@ -30,6 +31,12 @@ def _load():
         return None, str(e)
     if _autograd.torch_version != torch.__version__:
         return None, f"built for torch {_autograd.torch_version}, this is {torch.__version__}"
+    try:
+        torch.compiler.is_compiling, torch._C._are_functorch_transforms_active
+        torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+        forward_ad._current_level, torch._C._get_tracing_state
+    except AttributeError as e:
+        return None, str(e)
     L = _lib.load()
     _autograd.bind({name: ctypes.cast(getattr(L, name), ctypes.c_void_p).value
                     for name in _ENTRIES})

@@ -1,5 +1,6 @@
 """The native autograd nodes are an addition to the Python classes: the package
-imports without them, or with a module of another torch, and says so once."""
+imports without them, with a module of another torch, or in a torch without one of
+the private names that decide which calls are plain, and says so once."""
 import os
 import subprocess
 import sys
@@ -20,13 +21,29 @@ sys.modules["gs_voxelizer._autograd"] = m
 """
 
 
-@pytest.mark.parametrize("before,why", [(MISSING, "_autograd"), (OTHER_TORCH, "torch 1.0.0")],
-                         ids=["missing", "other_torch"])
+def _without(owner, name):
+    return (f"import torch, torch.autograd.forward_ad\nsaved = {owner}.{name}\n"
+            f"delattr({owner}, {name!r})\n"
+            f"restore = lambda: setattr({owner}, {name!r}, saved)  # torch itself uses some\n", name)
+
+
+@pytest.mark.parametrize("before,why", [
+    (MISSING, "_autograd"), (OTHER_TORCH, "torch 1.0.0"),
+    _without("torch._C", "_are_functorch_transforms_active"),
+    _without("torch._C", "_len_torch_dispatch_stack"),
+    _without("torch._C", "_len_torch_function_stack"),
+    _without("torch._C", "_get_tracing_state"),
+    _without("torch.autograd.forward_ad", "_current_level"),
+    _without("torch.compiler", "is_compiling")],
+    ids=["missing", "other_torch", "transforms", "dispatch", "function", "trace", "forward_mode",
+         "compile"])
 def test_the_package_imports_without_the_nodes(before, why):
     code = before + """
 import torch
 import gs_voxelizer.optim_to_render as o, gs_voxelizer.voxelize, gs_voxelizer.graph
 from gs_voxelizer import _native
+if "restore" in globals():
+    restore()
 assert not _native.available and not _native.plain(torch.zeros(1))
 z = torch.zeros((0, 3))
 try:
