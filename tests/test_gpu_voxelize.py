@@ -21,6 +21,7 @@ import torch
 import oracle as O
 from gs_voxelizer import synthetic as S
 from helpers import gpu_bin, l1_vol_grad, np32, oracle_project, report_close, small_config
+from test_gpu_tile_cull import _passing
 
 pytestmark = pytest.mark.gpu
 
@@ -343,22 +344,34 @@ def test_backward_gaussians_without_pairs_get_zero_gradients(device, mode):
 @pytest.mark.parametrize("channels", [1, 2, 3, 4])
 @pytest.mark.parametrize("vol,n", [((8, 8, 8), 1), ((8, 8, 8), 15), ((8, 8, 8), 17),
                                    ((8, 8, 8), 257), ((9, 17, 23), 24), ((9, 17, 23), 700),
-                                   ((24, 24, 24), 54), ((33, 31, 30), 2100)])
+                                   ((24, 24, 24), 54), ((33, 31, 30), 2100),
+                                   ((64, 64, 64), 2100), ((64, 64, 64), 4200),
+                                   ((64, 64, 64), 8000), ((24, 24, 24), 300)])
 def test_forward_waves_sharing_a_tile(device, vol, n, channels):
-    """Few tiles, so several waves share one tile's list (2 to 16 by the tile and
-    Gaussian counts; at least 16 pairs each): lists shorter than one share, of one
-    pair more than a share or a batch of 64, and ragged edge tiles.  Sums of up to
-    700 binary32 terms in another order differ by at most 700 * 2^-24 = 4e-5 of
-    their size: inside the suite's rel 1e-4."""
+    """Few tiles, so several waves share one tile's list (at least 16 pairs each), by
+    the tile and Gaussian counts: 8 and 16 at one tile with 15 and 17, 257
+    Gaussians, 16 at 18 tiles / 700 and 80 / 2100, 2 at 27 / 54, 8 at 27 / 300, 4
+    and 8 at 512 / 2100 and 4200, 8000 (1 Gaussian in one tile and 24 in 18 leave
+    one wave a tile, for comparison).  Lists shorter than one share, of one pair
+    more than a share or a batch of 64, and ragged edge tiles; each wave writes its
+    share's cull flags.  Sums of up to 700 binary32 terms in another order differ
+    by at most 700 * 2^-24 = 4e-5 of their size: inside the suite's rel 1e-4."""
     import gs_voxelizer.cuda as _C
     work = S.make_gaussians(small_config(1, n, vol=vol, channels=channels), seed=n + channels)
     p = _prepare(work, device)
     inten = work.intensities.numpy()
     ref, amb = O.voxelize_fwd(vol, p["rids"], p["rbins"], p["rpr"], p["rcn"], inten, with_amb=True)
-    live = torch.empty(p["I"], device=device, dtype=torch.uint8)
+    live = torch.full((p["I"],), 255, device=device, dtype=torch.uint8)
     out = _C.voxelize_forward(vol, p["ids"], p["bins"], p["pr"], p["cn"], p["w"].intensities,
                               pair_live=live)
     report_close("volume", np32(out), ref, RTOL, ATOL, amb)
+    flags = np32(live)
+    assert set(np.unique(flags)) <= {0, 1}  # every pair was flagged
+    tiles = np.repeat(np.arange(len(p["rbins"])), p["rbins"][:, 1] - p["rbins"][:, 0])
+    culled = np.nonzero(flags == 0)[0]
+    pr64, cn64, i64 = (a.astype(np.float64) for a in (np32(p["pr"]), np32(p["cn"]), inten))
+    for k in culled[::max(1, len(culled) // 300)]:
+        assert not _passing(work.cfg, pr64, cn64, i64, int(p["rids"][k]), int(tiles[k])), k
     # the lists in capacity-sized arrays give the same bits
     pad = torch.cat([p["ids"], torch.zeros(3 * p["I"] + 64, device=device, dtype=torch.int32)])
     again = _C.voxelize_forward(vol, pad, p["bins"], p["pr"], p["cn"], p["w"].intensities)
