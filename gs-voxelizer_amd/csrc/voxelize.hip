@@ -35,11 +35,11 @@
 //    the mode changes no result beyond denormal magnitudes.
 //  * Along a voxel row (fixed y, z) the quadratic form is
 //    s(dx) = R0 + dx*(R1 + A2*dx): two FMAs per voxel once R0, R1 are set up.
-//  * Forward: one 64-lane wave per tile, lane = one x-row of 8 voxels.  Per
-//    batch of 64 Gaussians each lane prepares one Gaussian's row constants into
-//    LDS; the wave then walks the live ones, reading each record with a
-//    uniform-address (broadcast) LDS read, so no VALU slot is spent on
-//    broadcasting.
+//  * Forward: one 64-lane wave per tile (up to 16 sharing its list where the
+//    volume has few tiles), lane = one x-row of 8 voxels.  Per batch of 64
+//    Gaussians each lane prepares one Gaussian's row constants into LDS; the
+//    wave then walks the live ones, reading each record with a uniform-address
+//    (broadcast) LDS read, so no VALU slot is spent on broadcasting.
 //  * Backward: one wave per bucket of 64 (tile, Gaussian) pairs, lane = one
 //    Gaussian; the tile's vol_grad is staged once in LDS and read row by row
 //    with broadcast reads.  Each lane accumulates its Gaussian's moments
@@ -1038,11 +1038,25 @@ constexpr int kStageTilesVerySparse = C == 1 ? 8 : 6;  // < kVerySparsePairs
 constexpr int64_t kSparsePairs = 64;
 constexpr int64_t kVerySparsePairs = 24;
 
-// The most waves of pairs whose backward is one launch: the waves that are
-// resident at once at the up to 235 VGPRs of k_vox_bwd with kRows > 1.  us for the
-// pairs and the rest pass, as two launches and as one: 280 waves (40 x 48 x 36 /
-// 2k) 22.5, 20.0; 980 (100 x 150 x 80 / 5k) 40.1, 26.7; 760 (its C = 2 scene of
-// fixed scales) 48.0, 28.1.
+// The most waves of pairs whose backward is one launch (its second workgroup row
+// takes what the rest launch would).  The one-launch kernels hold more registers
+// (146 against 103 VGPRs at C = 1, K = 3; 232 against 127 at C = 3, K = 2), and of
+// the up to 4,096 workgroups LDS keeps 1,024 at C = 3, K = 6 and 768 at C = 4, K =
+// 6, so a larger scene would pay for both.  Up to here the saved launch and its
+// gap are worth more.  us of the whole backward call as two launches and as one,
+// axes of 0.5-3 voxels:
+//   waves / pairs per tile   C = 1        C = 2        C = 3        C = 4
+//     300 / 150            29.5  27.7   34.1  32.2   36.4  34.7   39.7  37.9
+//    1000 / 87             32.4  30.8   52.7  35.9   57.9  45.3   66.4  48.5
+//    1000 / 47             33.3  31.6   38.7  37.0   41.4  46.7   47.0  46.2
+//    1000 / 12             47.2  32.8   75.9  46.1   85.9  62.6  130.5  80.7
+//    1500 / 131            39.2  37.4   47.6  45.4   51.1  49.9   59.0  55.6
+//    2000 / 176            43.0  42.6   51.2  52.4   54.4  53.2   63.2  59.6
+//    2000 / 46             43.3  42.5   67.0  54.3   73.2  71.3  100.6  80.0
+//    2000 / 12             69.5  48.9  141.0  78.1  156.7 109.1  215.0 161.6
+// Of 36 such scenes a channel count, three are slower by more than 2 %: C = 3 at
+// 1,000 waves of 47 and of 63 pairs per tile (K = 4: LDS holds 1,536 of the 2,000
+// workgroups) and C = 2 at 2,000 of 176.
 constexpr int64_t kSmallWaves = 2048;
 constexpr int kSmallRows = 2;
 
@@ -1547,9 +1561,10 @@ __device__ __forceinline__ void bwd_gaussian(const BwdArgs &a, BwdLane<C> &L) {
     const unsigned flags = (unsigned)__float_as_int(r0.w);
     L.off = r1.x;
     L.live = (flags & kRecLive) != 0;
-    // A work list holds only pairs the forward's identical test kept, so the
-    // test is not repeated for them (a pair it would cull has no passing
-    // voxel and yields zero moments either way).
+    // A work list holds the pairs that the forward's test kept (the second of
+    // this one's two, on the whole tile's box), so none is made for them here: a
+    // pair that this one would cull besides has no passing voxel and yields zero
+    // moments.
     if (L.live && (flags & kRecBounded) && a.order == nullptr) {
         const float2 c01 = a.conics[3 * g], c23 = a.conics[3 * g + 1], c45 = a.conics[3 * g + 2];
         L.live = may_touch(r0.x, r0.y, r0.z, c01.x, c01.y, c23.x, c23.y, c45.x, c45.y, r2.w,
@@ -1871,14 +1886,17 @@ __device__ __forceinline__ void zero_partial(const BwdArgs &a, int64_t e) {
 // the work list of kept pairs), lane = pair, so no lane idles except in the
 // last wave.  The wave stages the first K tiles its pairs span (lane = row;
 // each lane reads its own tile's rows); the pairs of further tiles are left to
-// k_vox_bwd_rest.  At C = 2 and 3 the kernel fits 128 VGPRs (4 waves per
-// SIMD), but left free the compiler's schedule for C = 2, K = 6 and C = 3,
-// K = 4 took all 256 and spilled into AGPRs (1 wave per SIMD): the bound
-// holds those two to the others' occupancy.  C = 1 (106 VGPRs) and C = 4
-// (3 waves) take the compiler's own choice.  C = 3, K = 6 stages 36,960 bytes,
-// which LDS holds to one wave per SIMD: there the bound only caps the
-// registers (128 VGPRs, no AGPRs), and the compiler's note that it missed the
-// occupancy target is silenced.
+// k_vox_bwd_rest.  Registers (kRows = 1): C = 1 takes 103 VGPRs (129 at K = 8),
+// C = 4 138 (219 at K = 4 and 6), both by the compiler's own choice.  At C = 2 and
+// 3 that choice took all 256 and spilled into AGPRs (1 wave per SIMD) for C = 2,
+// K = 6 and C = 3, K = 4, so they are bound to 2 waves per SIMD: 117 and 127 at
+// K = 2, 168 and 192 at K = 4 and 6, where LDS allows no more waves anyway (C = 3,
+// K = 6 stages 36,960 bytes, one wave per SIMD; the compiler's note that it missed
+// the occupancy target is silenced).  Against 114 to 142 VGPRs before the grouped
+// v_exp_f32 the sparse kernels did not get slower: 20,000 waves at 42 pairs per
+// tile 183 -> 181 us (C = 1), 266 -> 265 (2), 382 -> 383 (3), 615 -> 611 (4), at
+// 12 per tile 295 -> 275, 748 -> 561, 991 -> 845, 1,430 -> 1,273 (those mostly by
+// the rest pass's grid).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wpass-failed"
 //
@@ -2123,6 +2141,22 @@ int fwd_split(int64_t T, int64_t n) {
     return split;
 }
 
+// The backward's pass over `waves` waves of pairs: in one launch up to
+// kSmallWaves, else with the rest pass behind it.
+template <int C, int K>
+int launch_pairs(int64_t waves, const BwdArgs &args, hipStream_t s) {
+    const unsigned blocks = (unsigned)(kXcds * xcd_per(waves));
+    if (waves <= kSmallWaves) {
+        hipLaunchKernelGGL((k_vox_bwd<C, K, kSmallRows>), dim3(blocks, kSmallRows), dim3(kWave), 0,
+                           s, args);
+        return check_launch();
+    }
+    hipLaunchKernelGGL((k_vox_bwd<C, K, 1>), dim3(blocks), dim3(kWave), 0, s, args);
+    if (int st = check_launch()) return st;
+    hipLaunchKernelGGL((k_vox_bwd_rest<C, K>), dim3(rest_blocks(waves)), dim3(kWave), 0, s, args);
+    return check_launch();
+}
+
 // Forward; with `target`, also the L1 loss mean|volume - target| into *loss
 // (tile_loss: T floats of scratch) and sgn(volume - target) into sgn.
 int voxelize_fwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t n,
@@ -2237,7 +2271,6 @@ int voxelize_bwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t
     prep.rec = reinterpret_cast<float4 *>(ws + L.rec);
     const int nprep = (int)((n + kPrepThreads - 1) / kPrepThreads);
     const int64_t waves = (num_intersects + kWave - 1) / kWave;
-    const bool small = waves <= kSmallWaves;
     if (!pair_live) {
         const dim3 pgrid((unsigned)nprep), pblock(kPrepThreads);
         switch (channels) {
@@ -2280,8 +2313,6 @@ int voxelize_bwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t
         order = ord;
         d_work = kept;
     }
-    const int64_t per = xcd_per(waves);
-    const dim3 grid((unsigned)(kXcds * per)), block(kWave);
     const float numel = (float)((int64_t)D * H * W * channels);
     BwdArgs args;
     args.D = D; args.H = H; args.W = W; args.Tx = Tx; args.Ty = Ty; args.n = n; args.n_isect = ni;
@@ -2303,42 +2334,22 @@ int voxelize_bwd_impl(int32_t D, int32_t H, int32_t W, int32_t channels, int32_t
     args.d_work = d_work;
     args.n_work = 0;
     args.rest_flag = reinterpret_cast<uint8_t *>(ws + L.rest);
-#define GSV_VB(CH)                                                                                  \
-    {                                                                                               \
-        KernelTimer timer(kTimedVoxBwd, s);                                                         \
-        if (small) {                                                                                \
-            const dim3 rows(grid.x, kSmallRows);                                                    \
-            hipLaunchKernelGGL((very_sparse ? k_vox_bwd<CH, kStageTilesVerySparse<CH>, kSmallRows>  \
-                                : sparse    ? k_vox_bwd<CH, kStageTilesSparse<CH>, kSmallRows>      \
-                                            : k_vox_bwd<CH, kStageTiles<CH>, kSmallRows>),          \
-                               rows, block, 0, s, args);                                            \
-        } else if (very_sparse) {                                                                   \
-            hipLaunchKernelGGL((k_vox_bwd<CH, kStageTilesVerySparse<CH>, 1>), grid, block, 0, s,       \
-                               args);                                                               \
-            if (int st = check_launch()) return st;                                                 \
-            hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTilesVerySparse<CH>>),                     \
-                               dim3(rest_blocks(waves)), block, 0, s, args);                               \
-        } else if (sparse) {                                                                        \
-            hipLaunchKernelGGL((k_vox_bwd<CH, kStageTilesSparse<CH>, 1>), grid, block, 0, s, args);   \
-            if (int st = check_launch()) return st;                                                 \
-            hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTilesSparse<CH>>), dim3(rest_blocks(waves)),     \
-                               block, 0, s, args);                                                  \
-        } else {                                                                                    \
-            hipLaunchKernelGGL((k_vox_bwd<CH, kStageTiles<CH>, 1>), grid, block, 0, s, args);         \
-            if (int st = check_launch()) return st;                                                 \
-            hipLaunchKernelGGL((k_vox_bwd_rest<CH, kStageTiles<CH>>), dim3(rest_blocks(waves)), block, 0, \
-                               s, args);                                                            \
-        }                                                                                           \
-    }                                                                                               \
-    if (int st = check_launch()) return st;                                                         \
-    if (pairs) {                                                                                    \
-        KernelTimer timer(kTimedPairReduce, s);                                                     \
+#define GSV_VB(CH)                                                                                 \
+    {                                                                                              \
+        KernelTimer timer(kTimedVoxBwd, s);                                                        \
+        const int st =                                                                             \
+            very_sparse ? launch_pairs<CH, kStageTilesVerySparse<CH>>(waves, args, s)              \
+            : sparse    ? launch_pairs<CH, kStageTilesSparse<CH>>(waves, args, s)                  \
+                        : launch_pairs<CH, kStageTiles<CH>>(waves, args, s);                       \
+        if (st) return st;                                                                         \
+    }                                                                                              \
+    if (pairs) {                                                                                   \
+        KernelTimer timer(kTimedPairReduce, s);                                                    \
+        const int64_t lanes = (int64_t)n * kRowLanes;                                              \
         hipLaunchKernelGGL(k_pair_reduce<CH>,                                                      \
-                           dim3((unsigned)(((int64_t)n * kRowLanes + kReduceThreads - 1) /          \
-                                           kReduceThreads)),                                        \
+                           dim3((unsigned)((lanes + kReduceThreads - 1) / kReduceThreads)),        \
                            dim3(kReduceThreads), 0, s, n, ni, count_dev, args.rec, partial,        \
-                           conics, dpos3d_radii, dconics,                                           \
-                           dintensities);                                                           \
+                           conics, dpos3d_radii, dconics, dintensities);                           \
     }
     // pairs per tile from the count the grids are sized for (an upper bound
     // when the live count is on the device)
