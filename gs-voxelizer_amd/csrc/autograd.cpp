@@ -17,7 +17,6 @@
 #include <c10/hip/HIPStream.h>
 
 #include <atomic>
-#include <iterator>
 #include <map>
 #include <string>
 #include <tuple>
@@ -297,11 +296,13 @@ variable_list saved_tensors(const Tensor &pr, const Tensor &cn, const Tensor &in
         if (v.sign.defined()) return {pr, cn, intens, empty({0}, pr, at::kInt), v.bins, v.sign};
         return {pr, cn, intens, empty({0, 1}, pr, at::kInt), empty({0, 3}, pr, at::kInt)};
     }
-    variable_list saved{pr, cn, intens, v.ids.narrow(0, 0, v.count), v.bins};
-    if (v.sign.defined()) saved.push_back(v.sign);
-    const Tensor rest[] = {v.tile_min, v.tile_max, v.cum, v.tiles.narrow(0, 0, v.count), v.live};
-    saved.insert(saved.end(), std::begin(rest), std::end(rest));
-    return saved;
+    // (no other tensor shares these two, so they shrink in place, without views)
+    v.ids.unsafeGetTensorImpl()->set_sizes_contiguous({v.count});
+    v.tiles.unsafeGetTensorImpl()->set_sizes_contiguous({v.count});
+    if (v.sign.defined())
+        return {pr, cn, intens, v.ids, v.bins, v.sign, v.tile_min, v.tile_max, v.cum, v.tiles,
+                v.live};
+    return {pr, cn, intens, v.ids, v.bins, v.tile_min, v.tile_max, v.cum, v.tiles, v.live};
 }
 
 void remember(AutogradContext *ctx, const Volume &vol, const Voxelized &v, const Tensor &intens,
