@@ -297,7 +297,12 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 // At least six waves per SIMD at C = 1 (68 VGPRs, no spills, so seven; five and
-// eight, at 64, measured within 1 % of it); more channels would spill at six.
+// eight, at 64, measured within 1 % of it); more channels would spill at six.  At
+// most four at C = 3: the fifth that its 96 VGPRs leave room for gains at most 3 %
+// where rows are stored whole (364 -> 356 us at 301^3 / 400k), but the fused L1 on
+// an odd width reads, writes and signs rows element by element, and with five
+// waves the partial lines of a row leave the L2 before they are complete: 1,324 ->
+// 1,477 us at 378 x 340 x 289 / 120k, 958 -> 1,049 us at 301^3 / 60k.
 //
 // S waves per tile (fwd_split chooses S), each walking an equal share of the
 // tile's list, at least kMinShare pairs; wave 0 adds their sums in order and
@@ -306,7 +311,7 @@ constexpr int kMinShare = 16;  // 12 to 32 measured alike
 
 template <int C, int S>
 __global__ __launch_bounds__(kWave *S)
-__attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, 8))) void k_vox_fwd(
+__attribute__((amdgpu_waves_per_eu(C == 1 ? 6 : 1, C == 3 ? 4 : 8))) void k_vox_fwd(
     int D, int H, int W, int Tx, int Ty, int64_t T, int n, int n_isect,
     const int *__restrict__ ids, const int2 *__restrict__ bins, const float4 *__restrict__ pos_radii,
     const float2 *__restrict__ conics, const float *__restrict__ intens, float *__restrict__ vol,
