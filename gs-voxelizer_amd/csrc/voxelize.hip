@@ -195,7 +195,11 @@ __device__ __forceinline__ bool may_touch(float mx, float my, float mz, float a,
 // three v_exp_f32 together between priority changes, 1,189 with the v_exp_f32
 // replaced by moves.  k_vox_bwd: 336 -> 324 us at 256^3 / 200k, 133 -> 121 us at
 // 100 x 150 x 80 / 100k, 2.63 -> 2.54 ms at 512^3 / 1M.  The asm statements tie
-// the order to the values.
+// the order to the values.  Not in the kernels of very sparse scenes, whose LDS
+// share leaves a SIMD 3 waves or fewer, many of them waiting: the whole backward
+// took 269 -> 278 us at 281 x 341 x 262 / 11k, 200 -> 207 at 290 x 251 x 218 / 5k,
+// 178 -> 181 and 216 -> 219 at 200^3 / 20k at C = 2 and 3 (dense: 223 -> 213 at
+// 160^3 / 200k).
 __device__ __forceinline__ void exp2_together(float &x, float &y, float &z) {
     asm volatile("s_setprio 3" : "+v"(x), "+v"(y), "+v"(z));
     x = __builtin_amdgcn_exp2f(x);
@@ -878,7 +882,7 @@ __device__ __forceinline__ void row_centre(float al, float b2, float g3, double 
 //              indefinite and non-finite ones, as the reference evaluates it.
 constexpr int kRowsExact = 0, kRowsForm = 1, kRowsChain = 2;
 
-template <int C, int kMode>
+template <int C, int kMode, bool kTogether>
 __device__ __forceinline__ void pair_moments(const float4 *s_rows, float mxl, float myl, float mzl,
                                              const RowForm &f, float A2, float Bn, float Cn,
                                              float Dn, float En, float Fn, float shift, float bound,
@@ -947,7 +951,13 @@ __device__ __forceinline__ void pair_moments(const float4 *s_rows, float mxl, fl
                 float step = ur * (2.0f * f.al);       // 2^(2 al u_r)
                 float e1 = fmaf(ur, 2.0f * xu[0], q);  // u = 0
                 float e2 = fmaf(ur, 2.0f * xu[4], q);  // u = 4
-                exp2_together(step, e1, e2);
+                if (kTogether) {
+                    exp2_together(step, e1, e2);
+                } else {
+                    step = __builtin_amdgcn_exp2f(step);
+                    e1 = __builtin_amdgcn_exp2f(e1);
+                    e2 = __builtin_amdgcn_exp2f(e2);
+                }
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     sv[k] = e1 * G[k];
@@ -1678,6 +1688,7 @@ __device__ __forceinline__ void load_grad_row(const BwdArgs &a, int64_t off, int
 template <int C, int K>
 __device__ __forceinline__ void bwd_group(const BwdArgs &a, const BwdLane<C> &L, uint64_t starts,
                                           int g0, bool wave_fast, bool any_live, float4 *s_g) {
+    constexpr bool kTogether = K < kStageTilesVerySparse<C>;  // see exp2_together
     constexpr int kRowF4 = 2 * C;              // float4 per staged row
     constexpr int kSlot = kWave * kRowF4 + 1;  // +16 B: slots start on different banks
     const int lane = threadIdx.x;
@@ -1773,11 +1784,13 @@ __device__ __forceinline__ void bwd_group(const BwdArgs &a, const BwdLane<C> &L,
                     Gt[0] = r6.x; Gt[1] = r6.y; Gt[2] = r6.z; Gt[3] = r6.w;
                     Gt[4] = r7.x; Gt[5] = r7.y; Gt[6] = r7.z; Gt[7] = r7.w;
                 }
-                pair_moments<C, kRowsChain>(s_g + my * kSlot, gx, gy, gz, rf, 0.f, 0.f, 0.f, 0.f, 0.f,
-                                            0.f, 0.f, off, kshift, Gt, L.I, M);
+                pair_moments<C, kRowsChain, kTogether>(s_g + my * kSlot, gx, gy, gz, rf, 0.f, 0.f,
+                                                       0.f, 0.f, 0.f, 0.f, 0.f, off, kshift, Gt,
+                                                       L.I, M);
             } else {
-                pair_moments<C, kRowsForm>(s_g + my * kSlot, gx, gy, gz, rf, 0.f, 0.f, 0.f, 0.f, 0.f,
-                                           0.f, 0.f, off, 0.f, Gt, L.I, M);
+                pair_moments<C, kRowsForm, kTogether>(s_g + my * kSlot, gx, gy, gz, rf, 0.f, 0.f,
+                                                      0.f, 0.f, 0.f, 0.f, 0.f, off, 0.f, Gt, L.I,
+                                                      M);
             }
         } else {
             // lanes outside the group: a zero form, never inside the gate (|s| <= -1)
@@ -1792,8 +1805,9 @@ __device__ __forceinline__ void bwd_group(const BwdArgs &a, const BwdLane<C> &L,
             const float Cn = in_grp ? -kLog2e * c23.x : 0.f, Dn = in_grp ? -0.5f * kLog2e * c23.y : 0.f;
             const float En = in_grp ? -kLog2e * c45.x : 0.f, Fn = in_grp ? -0.5f * kLog2e * c45.y : 0.f;
             const float Gt[GSV_TILE] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};  // unused
-            pair_moments<C, kRowsExact>(s_g + my * kSlot, gx, gy, gz, RowForm{}, A2, Bn, Cn, Dn, En,
-                                        Fn, gt.shift, in_grp ? gt.half : -1.f, 0.f, Gt, L.I, M);
+            pair_moments<C, kRowsExact, kTogether>(s_g + my * kSlot, gx, gy, gz, RowForm{}, A2, Bn,
+                                                   Cn, Dn, En, Fn, gt.shift,
+                                                   in_grp ? gt.half : -1.f, 0.f, Gt, L.I, M);
         }
         __syncthreads();  // a later group restages the slots
     }
@@ -1891,17 +1905,15 @@ __device__ __forceinline__ void zero_partial(const BwdArgs &a, int64_t e) {
 // the work list of kept pairs), lane = pair, so no lane idles except in the
 // last wave.  The wave stages the first K tiles its pairs span (lane = row;
 // each lane reads its own tile's rows); the pairs of further tiles are left to
-// k_vox_bwd_rest.  Registers (kRows = 1): C = 1 takes 103 VGPRs (129 at K = 8),
-// C = 4 138 (219 at K = 4 and 6), both by the compiler's own choice.  At C = 2 and
-// 3 that choice took all 256 and spilled into AGPRs (1 wave per SIMD) for C = 2,
-// K = 6 and C = 3, K = 4, so they are bound to 2 waves per SIMD: 117 and 127 at
-// K = 2, 168 and 192 at K = 4 and 6, where LDS allows no more waves anyway (C = 3,
-// K = 6 stages 36,960 bytes, one wave per SIMD; the compiler's note that it missed
-// the occupancy target is silenced).  Against 114 to 142 VGPRs before the grouped
-// v_exp_f32 the sparse kernels did not get slower: 20,000 waves at 42 pairs per
-// tile 183 -> 181 us (C = 1), 266 -> 265 (2), 382 -> 383 (3), 615 -> 611 (4), at
-// 12 per tile 295 -> 275, 748 -> 561, 991 -> 845, 1,430 -> 1,273 (those mostly by
-// the rest pass's grid).
+// k_vox_bwd_rest.  Registers (kRows = 1): C = 1 takes 103 VGPRs (106 at K = 8),
+// C = 4 138 (219 at K = 4, 142 at 6), both by the compiler's own choice.  At C = 2
+// and 3 that choice took all 256 and spilled into AGPRs (1 wave per SIMD) for C =
+// 2, K = 6 and C = 3, K = 4, so they are bound to 2 waves per SIMD: 117 and 127 at
+// K = 2, 168 and 192 at K = 4, 114 and 127 at K = 6; at K = 4 and 6 LDS allows few
+// waves anyway (C = 3, K = 6 stages 36,960 bytes, one wave per SIMD; the compiler's
+// note that it missed the occupancy target is silenced).  With the grouped
+// v_exp_f32 K = 4 takes 53 to 77 VGPRs more, which costs it nothing: 20,000 waves
+// at 42 pairs per tile 266 -> 265 us (C = 2), 382 -> 383 (3), 615 -> 611 (4).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wpass-failed"
 //
