@@ -2138,23 +2138,39 @@ namespace gsv {
 namespace {
 
 // Waves per tile of the forward: with one, a volume of few tiles leaves most of
-// the chip's ~6,000 wave slots empty and its time is one tile's list, walked by
-// one wave.  The largest power of two that keeps the launch within about two
-// rounds of the slots and no more waves than Gaussians: an average Gaussian
-// reaches ~8 tiles and more, so their shares then average 8 pairs and more.  The
+// the chip's wave slots (4,096 at C = 3 and 4, 7,168 at C = 1) empty and its time
+// is one tile's list, walked by one wave.  The largest power of two at which the
+// launch either fits the slots with 1.5 Gaussians a wave, or stays within about
+// two rounds of them with 5: waves past a list's 16-pair shares have nothing to
+// do, which costs little beside empty slots and a round of its own otherwise.  The
 // rule takes nothing that differs between a count read on the host and one left
-// on the device, so the sums (their order depends on S and on the list alone)
-// are the same bits in both modes.  us at S = 1, 2, 4, 8 without the Gaussian
-// rule: 150 tiles of 103 pairs (2k Gaussians) 26.8, 18.5, 12.5, 10.6; 2,470 of
-// 495 (100k) 117, 94, 82, 84; 4,096 of 81 (50k) 35.5, 30.1, 31.9, 39.9; 2,470 of
-// 20 (5k) 14.0, 14.0, 16.5, 22.1; 11,960 of 143 (C = 3, 120k) 133, 132, 137, 189;
-// 32,768 of 108 (200k) 178, 178, 194, 275.
+// on the device, so the sums (their order depends on S and on the list alone) are
+// the same bits in both modes.  us at S = 1, 2, 4, 8:
+//   tiles  pairs / tile    Gaussians    C = 1                     C = 3
+//     512    13                1,228     6.5   6.2   6.2   6.3     7.6   7.3   7.3   7.4
+//     512    71                6,553    16.9  10.7   8.1   8.3    20.2  13.6   9.8  10.4
+//    1728    30                8,709    10.4   9.3   9.8  14.7    13.8  12.6  15.4  23.3
+//    2744    30               13,829    12.7  11.9  13.4  20.2    17.1  17.0  21.1  33.6
+//    2744    24               23,448    11.6  11.1  13.0  20.0    15.5  16.7  20.6  33.1
+//    2744   143               65,856    38.3  34.6  27.8  31.9    51.8  46.1  39.7  48.5
+//    4096    77               52,428    29.2  25.1  25.2  33.2    39.9  35.5  38.0  54.5
+// and 11,960 tiles of 143 (C = 3, 120k) 133, 132, 137, 189; 32,768 of 108 (200k)
+// 178, 178, 194, 275.  Over 972 scenes of 64 to 5,832 tiles, 4 to 300 pairs a tile
+// and 1 to 4 channels the forward takes 0.86 to 0.87 of its time at S = 1 on
+// average; 15 are slower than there, by at most 6 %.  With one Gaussian a wave up
+// to 12,288 waves it was 118 of them, by up to 52 % (2,744 tiles, C = 3).
+constexpr int64_t kSplitSlots = 4096;
 constexpr int64_t kSplitWaves = 12288;
 constexpr int kMaxSplit = 16;
 
 int fwd_split(int64_t T, int64_t n) {
     int split = 1;
-    while (split < kMaxSplit && 2 * split * T <= kSplitWaves && 2 * split * T <= n) split *= 2;
+    while (split < kMaxSplit) {
+        const int64_t waves = 2 * split * T;
+        const bool fits = waves <= kSplitSlots && 3 * waves <= 2 * n;
+        if (!fits && !(waves <= kSplitWaves && 5 * waves <= n)) break;
+        split *= 2;
+    }
     return split;
 }
 

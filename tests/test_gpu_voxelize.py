@@ -346,16 +346,18 @@ def test_backward_gaussians_without_pairs_get_zero_gradients(device, mode):
                                    ((8, 8, 8), 257), ((9, 17, 23), 24), ((9, 17, 23), 700),
                                    ((24, 24, 24), 54), ((33, 31, 30), 2100),
                                    ((64, 64, 64), 2100), ((64, 64, 64), 4200),
-                                   ((64, 64, 64), 8000), ((24, 24, 24), 300)])
+                                   ((64, 64, 64), 8000), ((24, 24, 24), 300),
+                                   ((104, 104, 104), 22000)])
 def test_forward_waves_sharing_a_tile(device, vol, n, channels):
     """Few tiles, so several waves share one tile's list (at least 16 pairs each), by
-    the tile and Gaussian counts: 8 and 16 at one tile with 15 and 17, 257
-    Gaussians, 16 at 18 tiles / 700 and 80 / 2100, 2 at 27 / 54, 8 at 27 / 300, 4
-    and 8 at 512 / 2100 and 4200, 8000 (1 Gaussian in one tile and 24 in 18 leave
-    one wave a tile, for comparison).  Lists shorter than one share, of one pair
-    more than a share or a batch of 64, and ragged edge tiles; each wave writes its
-    share's cull flags.  Sums of up to 700 binary32 terms in another order differ
-    by at most 700 * 2^-24 = 4e-5 of their size: inside the suite's rel 1e-4."""
+    the tile and Gaussian counts: 8 at one tile with 15 and 17 Gaussians and at 512
+    with 8000, 16 at one tile with 257, 18 with 700 and 80 with 2100, 4 at 27 with
+    300 and 512 with 4200, 2 at 512 with 2100 and 2197 with 22000 (1 Gaussian in
+    one tile, 24 in 18 and 54 in 27 leave one wave a tile, for comparison).  Lists
+    shorter than one share, of one pair more than a share or a batch of 64, and
+    ragged edge tiles; each wave writes its share's cull flags.  Sums of up to 700
+    binary32 terms in another order differ by at most 700 * 2^-24 = 4e-5 of their
+    size: inside the suite's rel 1e-4."""
     import gs_voxelizer.cuda as _C
     work = S.make_gaussians(small_config(1, n, vol=vol, channels=channels), seed=n + channels)
     p = _prepare(work, device)
