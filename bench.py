@@ -292,7 +292,7 @@ def main():
             roof["hbm_frac"] = round(roof["hbm_achieved_GBps"] / HBM_PEAK_GBS, 4)
     mem = _load_profile("mem", cfg.name)
     if mem is not None and mem.get("pairs") == n_isect:
-        k = mem["per_kernel"].get(f"k_vox_bwd<{C}, 3>") or next(
+        k = mem["per_kernel"].get(f"k_vox_bwd<{C}, 3, 1>") or next(
             (v for n, v in mem["per_kernel"].items() if n.startswith("k_vox_bwd<")), None)
         if k is not None:
             roof["wait_inst_any_frac"] = k["wait_inst_any_frac"]
