@@ -29,8 +29,11 @@ def _load():
         from . import _autograd
     except ImportError as e:  # not built, or against another torch's symbols
         return None, str(e)
-    if _autograd.torch_version != torch.__version__:
-        return None, f"built for torch {_autograd.torch_version}, this is {torch.__version__}"
+    built_for = getattr(_autograd, "torch_version", None)
+    if built_for is None:
+        return None, "_autograd.so is of an older build"
+    if built_for != torch.__version__:
+        return None, f"built for torch {built_for}, this is {torch.__version__}"
     try:
         torch.compiler.is_compiling, torch._C._are_functorch_transforms_active
         torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack

@@ -1,6 +1,7 @@
 """The native autograd nodes are an addition to the Python classes: the package
-imports without them, with a module of another torch, or in a torch without one of
-the private names that decide which calls are plain, and says so once."""
+imports without them, with a module of another torch or of an older build, or in a
+torch without one of the private names that decide which calls are plain, and says
+so once."""
 import os
 import subprocess
 import sys
@@ -19,6 +20,10 @@ m = types.ModuleType("gs_voxelizer._autograd")
 m.torch_version = "1.0.0"
 sys.modules["gs_voxelizer._autograd"] = m
 """
+OLDER_BUILD = """
+import sys, types
+sys.modules["gs_voxelizer._autograd"] = types.ModuleType("gs_voxelizer._autograd")
+"""
 
 
 def _without(owner, name):
@@ -28,15 +33,15 @@ def _without(owner, name):
 
 
 @pytest.mark.parametrize("before,why", [
-    (MISSING, "_autograd"), (OTHER_TORCH, "torch 1.0.0"),
+    (MISSING, "_autograd"), (OTHER_TORCH, "torch 1.0.0"), (OLDER_BUILD, "an older build"),
     _without("torch._C", "_are_functorch_transforms_active"),
     _without("torch._C", "_len_torch_dispatch_stack"),
     _without("torch._C", "_len_torch_function_stack"),
     _without("torch._C", "_get_tracing_state"),
     _without("torch.autograd.forward_ad", "_current_level"),
     _without("torch.compiler", "is_compiling")],
-    ids=["missing", "other_torch", "transforms", "dispatch", "function", "trace", "forward_mode",
-         "compile"])
+    ids=["missing", "other_torch", "older_build", "transforms", "dispatch", "function", "trace",
+         "forward_mode", "compile"])
 def test_the_package_imports_without_the_nodes(before, why):
     code = before + """
 import torch
